@@ -21,7 +21,7 @@ __global__ void __launch_bounds__(kFgThreads) k_fg_lines(double2* __restrict__ g
                                                          int n3, int axis, int nl, FftPlan pl,
                                                          const double* __restrict__ twtab,
                                                          int sign, double scale) {
-  extern __shared__ unsigned char smem_raw[];
+  extern __shared__ __align__(16) unsigned char smem_raw[];
   cplx<double>* tw = reinterpret_cast<cplx<double>*>(smem_raw);
   const int n = pl.n;
   cplx<double>* lines = tw + n;

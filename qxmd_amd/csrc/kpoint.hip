@@ -102,7 +102,7 @@ __global__ void __launch_bounds__(kKThreads)
 // one z plane of one (k, band) block; dynamic LDS: twiddles x | y, plane n2 x n1
 __global__ void __launch_bounds__(kKThreads)
     k_kplane(KArgs a, const double* __restrict__ V, double2* __restrict__ T) {
-  extern __shared__ unsigned char smem_raw[];
+  extern __shared__ __align__(16) unsigned char smem_raw[];
   cplx<double>* twx = reinterpret_cast<cplx<double>*>(smem_raw);
   cplx<double>* twy = twx + a.n1;
   cplx<double>* pl = twy + a.n2;

@@ -158,7 +158,7 @@ __device__ inline void pair_cols(int q0, int q1, int& c0, int& c1) {
 template <typename T>
 __global__ void __launch_bounds__(kZThreads) k_zinv(PencilArgs a, const double* __restrict__ psi,
                                                      cplx<T>* __restrict__ t1) {
-  extern __shared__ unsigned char smem_raw[];
+  extern __shared__ __align__(16) unsigned char smem_raw[];
   cplx<T>* tw = reinterpret_cast<cplx<T>*>(smem_raw);
   cplx<T>* lines = tw + a.n3;
   const int q0 = blockIdx.x * kPairsPerBlock;
@@ -200,7 +200,7 @@ template <typename T, typename VT>
 __global__ void __launch_bounds__(kPlaneThreads) k_plane(PencilArgs a, const VT* __restrict__ V,
                                                          const cplx<T>* __restrict__ t1,
                                                          cplx<T>* __restrict__ t2) {
-  extern __shared__ unsigned char smem_raw[];
+  extern __shared__ __align__(16) unsigned char smem_raw[];
   cplx<T>* twx = reinterpret_cast<cplx<T>*>(smem_raw);
   cplx<T>* twy = twx + a.n1;
   cplx<T>* A = twy + a.n2;                 // [nH][n2]
@@ -255,7 +255,7 @@ __global__ void __launch_bounds__(kZThreads) k_zfwd(PencilArgs a, const double* 
                                                      const cplx<T>* __restrict__ t2,
                                                      double* __restrict__ out, int accumulate,
                                                      double invN) {
-  extern __shared__ unsigned char smem_raw[];
+  extern __shared__ __align__(16) unsigned char smem_raw[];
   cplx<T>* tw = reinterpret_cast<cplx<T>*>(smem_raw);
   cplx<T>* lines = tw + a.n3;
   const int q0 = blockIdx.x * kPairsPerBlock;
@@ -310,7 +310,7 @@ __global__ void __launch_bounds__(kPlaneThreads) k_plane_rho(PencilArgs a, const
                                                              int nbp_batch, int bp_per_group,
                                                              const double* __restrict__ w,
                                                              double* __restrict__ rho_part) {
-  extern __shared__ unsigned char smem_raw[];
+  extern __shared__ __align__(16) unsigned char smem_raw[];
   cplx<T>* twx = reinterpret_cast<cplx<T>*>(smem_raw);
   cplx<T>* twy = twx + a.n1;
   cplx<T>* A = twy + a.n2;

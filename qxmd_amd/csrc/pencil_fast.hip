@@ -272,7 +272,7 @@ __global__ void __launch_bounds__(kPlaneMaxThreads) k_plane_f(FastArgs a, const 
   constexpr int N = NA * NB;
   constexpr int RW = plane_rows_per_wave(NA, NB);
   constexpr int NG = (N + RW - 1) / RW;
-  extern __shared__ unsigned char smem_raw[];
+  extern __shared__ __align__(16) unsigned char smem_raw[];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nwave = blockDim.x >> 6;
   const int sa = a.sa, sr = a.sr, nH = a.nH;
   cplx<T>* tw = reinterpret_cast<cplx<T>*>(smem_raw);
@@ -296,15 +296,17 @@ __global__ void __launch_bounds__(kPlaneMaxThreads) k_plane_f(FastArgs a, const 
     for (int kb = 0; kb < NB; ++kb) vv[kb] = row[kb];
   }
 
-  // sphere columns of this plane: loads issued before the LDS fill
+  // sphere columns of this plane: loads issued before the LDS fill (real and
+  // imaginary parts apart: an array of FP64 pairs went through scratch memory)
   const cplx<T>* in = t1 + ((size_t)bp * N + zs) * a.ncol;
-  cplx<T> cv[kPlaneLoads];
+  T cr[kPlaneLoads], cim[kPlaneLoads];
   int ci[kPlaneLoads];
 #pragma unroll
   for (int j = 0; j < kPlaneLoads; ++j) {
     const int cl = threadIdx.x + j * blockDim.x;
     const int cc = cl < a.ncol ? cl : 0;
-    cv[j] = in[cc];
+    cr[j] = in[cc].x;
+    cim[j] = in[cc].y;
     ci[j] = cl < a.ncol ? a.col_hi[cc] * sa + a.col_kmod[cc] : -1;
   }
   for (int k = threadIdx.x; k < N; k += blockDim.x) tw[k] = mk<T>((T)a.tw[2 * k], (T)a.tw[2 * k + 1]);
@@ -314,7 +316,7 @@ __global__ void __launch_bounds__(kPlaneMaxThreads) k_plane_f(FastArgs a, const 
   x_twiddles<T, NA, NB>(tw, jx, xw);
 #pragma unroll
   for (int j = 0; j < kPlaneLoads; ++j)
-    if (ci[j] >= 0) A[ci[j]] = cv[j];
+    if (ci[j] >= 0) A[ci[j]] = mk<T>(cr[j], cim[j]);
   for (int cl = threadIdx.x + kPlaneLoads * blockDim.x; cl < a.ncol; cl += blockDim.x)
     A[a.col_hi[cl] * sa + a.col_kmod[cl]] = in[cl];
   __syncthreads();
@@ -466,7 +468,7 @@ __global__ void __launch_bounds__(rho_max_threads(RG)) k_plane_rho_f(FastArgs a,
   constexpr int N = NA * NB;
   constexpr int RW = plane_rows_per_wave(NA, NB);
   constexpr int NG = (N + RW - 1) / RW;
-  extern __shared__ unsigned char smem_raw[];
+  extern __shared__ __align__(16) unsigned char smem_raw[];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nwave = blockDim.x >> 6;
   const int sa = a.sa, sr = a.sr, nH = a.nH;
   cplx<T>* tw = reinterpret_cast<cplx<T>*>(smem_raw);
