@@ -25,6 +25,8 @@ HIP_SOURCES = ["pencil.hip", "pencil_fast.hip", "gemm.hip", "mfma_gemm.hip", "bl
                "eigh.hip",
                "fullgrid.hip", "kpoint.hip", "cg.hip", "nlsetup.hip", "kb1.hip", "forces.hip", "flocal.hip", "ewald.hip",
                "aspc.hip", "scfglue.hip", "api.hip"]
+# compiled once per group of FFT edges (pencil_fast.h, kFftGroups)
+FFT_SOURCE, FFT_GROUPS = "pencil_inst.hip", 8
 HOST_SOURCES = ["gsphere.cpp", "restart.cpp", "mdstep.cpp"]
 FORTRAN_SOURCES = ["qxmd_amd_c.f90", "qxmd_dropin.f90"]
 FOUT = os.path.join(HERE, "libqxmd_amd_f.so")
@@ -56,6 +58,11 @@ def build(verbose: bool = False, jobs: int = 8) -> str:
     hipcc = _hipcc()
     cmds = []
     objs = []
+    for g in range(FFT_GROUPS):  # the longest compilations first
+        o = os.path.join(BLD, FFT_SOURCE.replace(".hip", f"_{g}.o"))
+        cmds.append([hipcc, *HIPCC_FLAGS, f"-DQX_FFT_GROUP={g}", "-c",
+                     os.path.join(CSRC, FFT_SOURCE), "-o", o])
+        objs.append(o)
     for s in HIP_SOURCES:
         o = os.path.join(BLD, s.replace(".hip", ".o"))
         cmds.append([hipcc, *HIPCC_FLAGS, "-c", os.path.join(CSRC, s), "-o", o])

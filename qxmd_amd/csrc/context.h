@@ -204,6 +204,7 @@ int pencil_build(Ctx* c, const int* nga, const int* ngb, const int* ngc, const d
 int local_apply(Ctx* c, const double* psi, double* out, int nb, int prec, int accumulate);
 int density(Ctx* c, const double* psi, int nb, const double* occ_dev, double scale, int prec);
 bool fast_ok(const Ctx* c);
+bool fast_split(int n, int* na, int* nb);
 int fast_permute_v(Ctx* c);
 int local_apply_fast(Ctx* c, const double* psi, double* out, int nb, int prec, int accumulate);
 int density_fast(Ctx* c, const double* psi, int nb, const double* w, int prec);

@@ -439,7 +439,7 @@ static int local_apply_t(Ctx* c, const double* psi, double* out, int nb, int acc
 }
 
 int local_apply(Ctx* c, const double* psi, double* out, int nb, int prec, int accumulate) {
-  if (fast_ok(c)) {
+  if (fast_ok(c) && c->d_Vp) {
     const int rc = local_apply_fast(c, psi, out, nb, prec, accumulate);
     if (rc != -3) return rc;  // -3: the fast plane kernel does not fit this grid
   }
