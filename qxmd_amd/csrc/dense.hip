@@ -456,6 +456,7 @@ static int chol_inv_legacy(Ctx* c, double* s, int n, double* x, int* flag) {
 // L^-1; ok[0] = lcholesky, ok[1] = 1 if a grid barrier gave up.  flag:
 // device int scratch.
 int dense_chol_inv(Ctx* c, double* s, int n, double* x, int* ok, int* flag) {
+  if (dense_wg_ok(n)) return chol_inv_wg(c, s, n, x, ok);
   hipStream_t st = c->stream;
   hipLaunchKernelGGL(k_flag_clear, dim3(1), dim3(1), 0, st, flag);
   const int nblk = (n + NBK - 1) / NBK;

@@ -922,15 +922,20 @@ int dense_eigh(Ctx* c, double* a, int n, double* z, double* w, double* work, int
   double* gram = X + (size_t)n * n;                             // n^2
   double* linv = gram + (size_t)n * n;                          // n^2
   double* lu = linv + (size_t)n * n;                            // 5 n^2
-  // 1. tridiagonalisation: the row distribution follows the group count, so
-  // the launch must get exactly the groups its LDS is sized for
+  // 1. tridiagonalisation, in one workgroup up to the order it holds; above,
+  // the row distribution follows the group count, so the launch must get
+  // exactly the groups its LDS is sized for
+  const bool one_wg = dense_wg_ok(n);
+  if (one_wg) {
+    if (int rc = tridiag_wg(c, a, n, d, e)) return rc;
+  }
   int dev = 0, ncu = 0;
   QX_CHECK(hipGetDevice(&dev));
   QX_CHECK(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev));
   const int G = std::min(tridiag_groups(n), std::min(n, ncu));
   const size_t rpw = (size_t)((n + G - 1) / G);
   const size_t lds = sizeof(double) * (rpw * n + (size_t)n + rpw + 24);
-  if (lds > 160 * 1024 - 1024 || n > 256 * kTrdM || G > 64 * kTrdKq)
+  if (!one_wg && (lds > 160 * 1024 - 1024 || n > 256 * kTrdM || G > 64 * kTrdKq))
     return dense_eigh_legacy(c, a, n, z, w, work);
   int* bar = c->d_sync;
   int* err = c->d_sync + 1;
@@ -938,14 +943,17 @@ int dense_eigh(Ctx* c, double* a, int n, double* z, double* w, double* work, int
   // idle until step 3; tags must start cleared
   unsigned long long* pub = reinterpret_cast<unsigned long long*>(X);
   const long npub = 8 * (long)n + 4 * (long)G;
-  hipLaunchKernelGGL(k_zero_u64, dim3((unsigned)((npub + 255) / 256)), dim3(256), 0, st, pub, npub);
+  if (!one_wg)
+    hipLaunchKernelGGL(k_zero_u64, dim3((unsigned)((npub + 255) / 256)), dim3(256), 0, st, pub,
+                       npub);
   void* args[] = {&a, &n, &d, &e, &rowbuf, &pub, &bar, &err};
   const void* trd =
       n <= 256 * 3 ? (G <= 64 * 3 ? reinterpret_cast<const void*>(k_tridiag_coop<3, 3>)
                                   : reinterpret_cast<const void*>(k_tridiag_coop<3, kTrdKq>))
       : n <= 256 * 5 ? reinterpret_cast<const void*>(k_tridiag_coop<5, kTrdKq>)
                      : reinterpret_cast<const void*>(k_tridiag_coop<kTrdM, kTrdKq>);
-  if (coop_launch(c, trd, G, lds, args, true) < 0) return dense_eigh_legacy(c, a, n, z, w, work);
+  if (!one_wg && coop_launch(c, trd, G, lds, args, true) < 0)
+    return dense_eigh_legacy(c, a, n, z, w, work);
   // 2. eigenvalues
   hipLaunchKernelGGL(k_gersh, dim3(1), dim3(256), 0, st, d, e, n, bounds);
   hipLaunchKernelGGL(k_bisect_ms, dim3((n + 3) / 4), dim3(256), 0, st, d, e, n, bounds, w);
