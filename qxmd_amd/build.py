@@ -21,7 +21,7 @@ OUT = os.path.join(HERE, "libqxmd_amd.so")
 BLD = os.path.join(HERE, "_build")
 ARCH = os.environ.get("QX_OFFLOAD_ARCH", "gfx950")
 
-HIP_SOURCES = ["pencil.hip", "pencil_fast.hip", "gemm.hip", "mfma_gemm.hip", "blaslt.hip", "dense.hip",
+HIP_SOURCES = ["pencil.hip", "pencil_fast.hip", "gemm.hip", "gemm_small.hip", "mfma_gemm.hip", "blaslt.hip", "dense.hip", "dense_small.hip",
                "eigh.hip",
                "fullgrid.hip", "kpoint.hip", "cg.hip", "nlsetup.hip", "kb1.hip", "forces.hip", "flocal.hip", "ewald.hip",
                "aspc.hip", "scfglue.hip", "api.hip"]

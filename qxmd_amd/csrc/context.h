@@ -85,6 +85,8 @@ struct Ctx {
   double *d_scal = nullptr;               // scalar work (device)
   int* d_sync = nullptr;                  // grid-barrier counter and error flags
   double* d_dwork = nullptr;              // dense eigensolver work (8 nbmax^2 + ...)
+  double* d_gs = nullptr;                 // K-slice partials of the small products
+  size_t gs_len = 0;
   double* d_bb = nullptr;                 // band-by-band CG: scalars, then chunk sums
   int bb_nch = 0;                         // chunks of kBbChunk the chunk-sum space holds
   int *h_flag = nullptr, *d_hflag = nullptr;  // pinned host flag and its device address
@@ -377,10 +379,24 @@ int flocal_host(Ctx* c, double* floc, int ntype, const int* nhk1, const int* nhk
                 const double* const* dcq, const double* const* dsq);
 int coop_launch(Ctx* c, const void* fn, int want, size_t lds, void** args, bool exact);
 int dense_chol_inv(Ctx* c, double* s, int n, double* x, int* ok, int* flag);
+// the same and the tridiagonalisation in one workgroup (dense_small.hip)
+bool dense_wg_ok(int n);
+int chol_inv_wg(Ctx* c, const double* s, int n, double* x, int* ok);
+int tridiag_wg(Ctx* c, double* a, int n, double* d, double* e);
 int gemm_tn(Ctx* c, int M, int N, int K, double alpha, const double* A, int lda, const double* B,
             int ldb, double beta, double* C, int ldc, int corr);
 int gemm_nn(Ctx* c, int M, int N, int K, double alpha, const double* A, int lda, const double* B,
             int ldb, double beta, double* C, int ldc);
+// the products with a dimension of the output below 256 (gemm_small.hip), in
+// either precision, over `batch` operands at the given strides; rscale: a
+// factor per row m of C (TN)
+int gs_gemm_tn(Ctx* c, int M, int N, int K, double alpha, const double* A, int lda, const double* B,
+               int ldb, double beta, double* C, int ldc, int corr, int prec,
+               const double* rscale = nullptr, int batch = 1, long sA = 0, long sB = 0,
+               long sC = 0);
+int gs_gemm_nn(Ctx* c, int M, int N, int K, double alpha, const double* A, int lda, const double* B,
+               int ldb, double beta, double* C, int ldc, int prec, int batch = 1, long sA = 0,
+               long sB = 0, long sC = 0);
 // the same contractions with a precision: PREC_FP32 -> FP32 MFMA (operands
 // rounded to FP32, FP32 accumulation per K chunk), otherwise FP64
 int gemm_tn_p(Ctx* c, int M, int N, int K, double alpha, const double* A, int lda,

@@ -15,11 +15,8 @@
 // which skips Im c(G=0): Sources/nlkbpp.f90:1360-1363).
 //
 // Sizable outputs (M, N >= 256) run on the 128 x 128 kernels of
-// mfma_gemm.hip.  The kernels here take the skinny shapes: 64x64 per
-// 256-thread block, 4 wavefronts of 32x32, each a 2x2 grid of
-// v_mfma_f64_16x16x4 blocks, K staged through LDS 16 at a time, the long-K
-// shape split over blocks and reduced with FP64 atomics; at most 4 columns,
-// matrix-vector kernels.
+// mfma_gemm.hip, smaller ones on gemm_small.hip, at most 4 columns on the
+// matrix-vector kernels here.
 #include <algorithm>
 #include <atomic>
 #include <cstdlib>
@@ -43,104 +40,6 @@ int gemm_path() {
 void set_gemm_path(int p) { g_gemm_path.store(p, std::memory_order_relaxed); }
 
 typedef double d4 __attribute__((ext_vector_type(4)));
-
-constexpr int BM = 64, BN = 64, KT = 16, LDT = BM + 2;
-
-template <bool AKC, bool SPLIT>
-__global__ void __launch_bounds__(256) k_gemm_f64(int M, int N, int K, int kchunk, double alpha,
-                                                  const double* __restrict__ A, int lda,
-                                                  const double* __restrict__ B, int ldb,
-                                                  double* __restrict__ C, int ldc) {
-  __shared__ double As[KT][LDT];
-  __shared__ double Bs[KT][LDT];
-  const int m0 = blockIdx.x * BM, n0 = blockIdx.y * BN;
-  const int kb = blockIdx.z * kchunk, ke = min(K, kb + kchunk);
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = (wave & 1) * 32, wn = (wave >> 1) * 32;
-  d4 acc[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = d4{0.0, 0.0, 0.0, 0.0};
-
-  // operands of a stage: unconditional loads from clamped (valid) addresses,
-  // then a select, so all of them are in flight together; the next stage is
-  // fetched into registers while the current one is on the MFMA pipes
-  double ra[4], rb[4];
-  auto fetch = [&](int k0) {
-    if (AKC) {
-      const int m = tid >> 2, kk = (tid & 3) * 4, gm = m0 + m, gmc = min(gm, M - 1);
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int gk = k0 + kk + u;
-        const double v = A[(size_t)gmc * lda + min(gk, ke - 1)];
-        ra[u] = (gm < M && gk < ke) ? v : 0.0;
-      }
-    } else {
-      const int kk = tid >> 4, m = (tid & 15) * 4, gk = k0 + kk, gkc = min(gk, ke - 1);
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int gm = m0 + m + u;
-        const double v = A[(size_t)gkc * lda + min(gm, M - 1)];
-        ra[u] = (gm < M && gk < ke) ? v : 0.0;
-      }
-    }
-    const int n = tid >> 2, kk = (tid & 3) * 4, gn = n0 + n, gnc = min(gn, N - 1);
-#pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int gk = k0 + kk + u;
-      const double v = B[(size_t)gnc * ldb + min(gk, ke - 1)];
-      rb[u] = (gn < N && gk < ke) ? v : 0.0;
-    }
-  };
-  fetch(kb);
-  for (int k0 = kb; k0 < ke; k0 += KT) {
-    if (AKC) {
-      const int m = tid >> 2, kk = (tid & 3) * 4;
-#pragma unroll
-      for (int u = 0; u < 4; ++u) As[kk + u][m] = ra[u];
-    } else {
-      const int kk = tid >> 4, m = (tid & 15) * 4;
-#pragma unroll
-      for (int u = 0; u < 4; ++u) As[kk][m + u] = ra[u];
-    }
-    {
-      const int n = tid >> 2, kk = (tid & 3) * 4;
-#pragma unroll
-      for (int u = 0; u < 4; ++u) Bs[kk + u][n] = rb[u];
-    }
-    __syncthreads();
-    if (k0 + KT < ke) fetch(k0 + KT);
-#pragma unroll
-    for (int k4 = 0; k4 < KT; k4 += 4) {
-      const int kr = k4 + (lane >> 4), c = lane & 15;
-      double a0 = As[kr][wm + c], a1 = As[kr][wm + 16 + c];
-      double b0 = Bs[kr][wn + c], b1 = Bs[kr][wn + 16 + c];
-      acc[0][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b0, acc[0][0], 0, 0, 0);
-      acc[0][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b1, acc[0][1], 0, 0, 0);
-      acc[1][0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b0, acc[1][0], 0, 0, 0);
-      acc[1][1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b1, acc[1][1], 0, 0, 0);
-    }
-    __syncthreads();
-  }
-  // ---- epilogue: v_mfma_f64_16x16x4 leaves D(i, j) in lane j + 16*(i%4),
-  // register i/4, i.e. acc[i][j][v] = C(m = .. + lane/16 + 4*v, n = .. + lane%16)
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      int n = n0 + wn + j * 16 + (lane & 15);
-      if (n >= N) continue;
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        int m = m0 + wm + i * 16 + (lane >> 4) + 4 * v;
-        if (m >= M) continue;
-        double val = alpha * acc[i][j][v];
-        if (SPLIT) atomicAdd(&C[(size_t)n * ldc + m], val);
-        else C[(size_t)n * ldc + m] += val;
-      }
-    }
-}
 
 __global__ void k_scale(double* C, int M, int N, int ldc, double beta) {
   long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -186,26 +85,10 @@ static int gemm_tn_small(Ctx* c, int M, int N, int K, double alpha, const double
     QX_CHECK(hipGetLastError());
     return 0;
   }
-  hipLaunchKernelGGL(k_scale, dim3(cdiv((long)M * N, 256)), dim3(256), 0, c->stream, C, M, N, ldc,
-                     beta);
-  const int tiles = (int)(cdiv(M, BM) * cdiv(N, BN));
-  int nsplit = std::max<int>(1, std::min<int>((int)cdiv(K, 1024), std::max(1, 2048 / tiles)));
-  int kchunk = (int)(cdiv(cdiv(K, nsplit), KT) * KT);
-  nsplit = (int)cdiv(K, kchunk);
-  dim3 grid(cdiv(M, BM), cdiv(N, BN), nsplit);
   lt_mark(c, c->lt_gemm_id, false);
-  if (nsplit > 1)
-    hipLaunchKernelGGL((k_gemm_f64<true, true>), grid, dim3(256), 0, c->stream, M, N, K, kchunk,
-                       alpha, A, lda, B, ldb, C, ldc);
-  else
-    hipLaunchKernelGGL((k_gemm_f64<true, false>), grid, dim3(256), 0, c->stream, M, N, K, kchunk,
-                       alpha, A, lda, B, ldb, C, ldc);
+  const int rc = gs_gemm_tn(c, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, corr, PREC_FP64);
   lt_mark(c, c->lt_gemm_id, true);
-  if (corr)
-    hipLaunchKernelGGL(k_corr, dim3(cdiv((long)M * N, 256)), dim3(256), 0, c->stream, C, M, N, ldc,
-                       A, lda, B, ldb, alpha, corr == 2 ? 1 : 0);
-  QX_CHECK(hipGetLastError());
-  return 0;
+  return rc;
 }
 
 static int gemm_nn_small(Ctx* c, int M, int N, int K, double alpha, const double* A, int lda,
@@ -216,16 +99,10 @@ static int gemm_nn_small(Ctx* c, int M, int N, int K, double alpha, const double
     QX_CHECK(hipGetLastError());
     return 0;
   }
-  if (beta != 1.0)
-    hipLaunchKernelGGL(k_scale, dim3(cdiv((long)M * N, 256)), dim3(256), 0, c->stream, C, M, N,
-                       ldc, beta);
-  dim3 grid(cdiv(M, BM), cdiv(N, BN), 1);
   lt_mark(c, c->lt_gemm_id, false);
-  hipLaunchKernelGGL((k_gemm_f64<false, false>), grid, dim3(256), 0, c->stream, M, N, K, K, alpha,
-                     A, lda, B, ldb, C, ldc);
+  const int rc = gs_gemm_nn(c, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, PREC_FP64);
   lt_mark(c, c->lt_gemm_id, true);
-  QX_CHECK(hipGetLastError());
-  return 0;
+  return rc;
 }
 
 // ---- skinny shapes (N <= 4 columns): matrix-vector products at HBM speed ---
@@ -355,103 +232,7 @@ static int gemv_nn(Ctx* c, int M, int N, int K, double alpha, const double* A, i
   return 0;
 }
 
-// ---- mixed precision: FP64 operands rounded to FP32 while staged into LDS,
-// v_mfma_f32_16x16x4f32 products with FP32 accumulation over each K chunk,
-// chunks combined in FP64 (split-K atomics or the FP64 C update).
 typedef float f4 __attribute__((ext_vector_type(4)));
-constexpr int KT32 = 32, LDT32 = BM + 4;
-
-template <bool AKC, bool SPLIT>
-__global__ void __launch_bounds__(256) k_gemm_f32(int M, int N, int K, int kchunk, double alpha,
-                                                  const double* __restrict__ A, int lda,
-                                                  const double* __restrict__ B, int ldb,
-                                                  double* __restrict__ C, int ldc) {
-  __shared__ float As[KT32][LDT32];
-  __shared__ float Bs[KT32][LDT32];
-  const int m0 = blockIdx.x * BM, n0 = blockIdx.y * BN;
-  const int kb = blockIdx.z * kchunk, ke = min(K, kb + kchunk);
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = (wave & 1) * 32, wn = (wave >> 1) * 32;
-  f4 acc[2][2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = f4{0.f, 0.f, 0.f, 0.f};
-  // per thread: 8 A values and 8 B values of the 64 x 32 stage
-  float ra[8], rb[8];
-  auto fetch = [&](int k0) {
-    if (AKC) {
-      const int m = tid >> 2, kk = (tid & 3) * 8, gm = m0 + m, gmc = min(gm, M - 1);
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const int gk = k0 + kk + u;
-        const double v = A[(size_t)gmc * lda + min(gk, ke - 1)];
-        ra[u] = (gm < M && gk < ke) ? (float)v : 0.f;
-      }
-    } else {
-      const int kk = tid >> 3, m = (tid & 7) * 8, gk = k0 + kk, gkc = min(gk, ke - 1);
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        const int gm = m0 + m + u;
-        const double v = A[(size_t)gkc * lda + min(gm, M - 1)];
-        ra[u] = (gm < M && gk < ke) ? (float)v : 0.f;
-      }
-    }
-    const int n = tid >> 2, kk = (tid & 3) * 8, gn = n0 + n, gnc = min(gn, N - 1);
-#pragma unroll
-    for (int u = 0; u < 8; ++u) {
-      const int gk = k0 + kk + u;
-      const double v = B[(size_t)gnc * ldb + min(gk, ke - 1)];
-      rb[u] = (gn < N && gk < ke) ? (float)v : 0.f;
-    }
-  };
-  fetch(kb);
-  for (int k0 = kb; k0 < ke; k0 += KT32) {
-    if (AKC) {
-      const int m = tid >> 2, kk = (tid & 3) * 8;
-#pragma unroll
-      for (int u = 0; u < 8; ++u) As[kk + u][m] = ra[u];
-    } else {
-      const int kk = tid >> 3, m = (tid & 7) * 8;
-#pragma unroll
-      for (int u = 0; u < 8; ++u) As[kk][m + u] = ra[u];
-    }
-    {
-      const int n = tid >> 2, kk = (tid & 3) * 8;
-#pragma unroll
-      for (int u = 0; u < 8; ++u) Bs[kk + u][n] = rb[u];
-    }
-    __syncthreads();
-    if (k0 + KT32 < ke) fetch(k0 + KT32);  // next stage in flight during the MFMAs
-#pragma unroll
-    for (int k4 = 0; k4 < KT32; k4 += 4) {
-      const int kr = k4 + (lane >> 4), c = lane & 15;
-      const float a0 = As[kr][wm + c], a1 = As[kr][wm + 16 + c];
-      const float b0 = Bs[kr][wn + c], b1 = Bs[kr][wn + 16 + c];
-      acc[0][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a0, b0, acc[0][0], 0, 0, 0);
-      acc[0][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a0, b1, acc[0][1], 0, 0, 0);
-      acc[1][0] = __builtin_amdgcn_mfma_f32_16x16x4f32(a1, b0, acc[1][0], 0, 0, 0);
-      acc[1][1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a1, b1, acc[1][1], 0, 0, 0);
-    }
-    __syncthreads();
-  }
-  // v_mfma_f32_16x16x4f32 leaves D(i, j) in lane j + 16*(i/4), register i%4
-#pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-      const int n = n0 + wn + j * 16 + (lane & 15);
-      if (n >= N) continue;
-#pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        const int m = m0 + wm + i * 16 + 4 * (lane >> 4) + v;
-        if (m >= M) continue;
-        const double val = alpha * (double)acc[i][j][v];
-        if (SPLIT) atomicAdd(&C[(size_t)n * ldc + m], val);
-        else C[(size_t)n * ldc + m] += val;
-      }
-    }
-}
 
 // ---- 128 x 128 tiles: four wavefronts of 64 x 64 (4 x 4 MFMA blocks each),
 // the next K stage fetched into registers while the current one is on the
@@ -617,7 +398,7 @@ static void launch_big_nn(Ctx* c, int M, int N, int K, double alpha, const doubl
 }
 
 // FP32-class contractions (the mixed form): our split bf16x3 MFMA kernels
-// for sizable outputs, FP32 MFMA tiles for skinny ones; hipBLASLt only as a
+// for sizable outputs, FP32 MFMA (gemm_small.hip) for others; hipBLASLt only as a
 // cross-check (QX_GEMM_LIB=hipblaslt)
 int gemm_tn_p(Ctx* c, int M, int N, int K, double alpha, const double* A, int lda, const double* B,
               int ldb, double beta, double* C, int ldc, int corr, int prec) {
@@ -639,24 +420,15 @@ int gemm_tn_p(Ctx* c, int M, int N, int K, double alpha, const double* A, int ld
     }
   }
 
+  lt_mark(c, c->lt_gemm_id, false);
+  if (!use_big(M, N)) {
+    const int rc = gs_gemm_tn(c, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, corr, PREC_FP32);
+    lt_mark(c, c->lt_gemm_id, true);
+    return rc;
+  }
   hipLaunchKernelGGL(k_scale, dim3(cdiv((long)M * N, 256)), dim3(256), 0, c->stream, C, M, N, ldc,
                      beta);
-  lt_mark(c, c->lt_gemm_id, false);
-  if (use_big(M, N)) {
-    launch_big_tn<float>(c, M, N, K, alpha, A, lda, B, ldb, C, ldc);
-  } else {
-    const int tiles = (int)(cdiv(M, BM) * cdiv(N, BN));
-    int nsplit = std::max<int>(1, std::min<int>((int)cdiv(K, 1024), std::max(1, 2048 / tiles)));
-    int kchunk = (int)(cdiv(cdiv(K, nsplit), KT32) * KT32);
-    nsplit = (int)cdiv(K, kchunk);
-    dim3 grid(cdiv(M, BM), cdiv(N, BN), nsplit);
-    if (nsplit > 1)
-      hipLaunchKernelGGL((k_gemm_f32<true, true>), grid, dim3(256), 0, c->stream, M, N, K, kchunk,
-                         alpha, A, lda, B, ldb, C, ldc);
-    else
-      hipLaunchKernelGGL((k_gemm_f32<true, false>), grid, dim3(256), 0, c->stream, M, N, K,
-                         kchunk, alpha, A, lda, B, ldb, C, ldc);
-  }
+  launch_big_tn<float>(c, M, N, K, alpha, A, lda, B, ldb, C, ldc);
   lt_mark(c, c->lt_gemm_id, true);
   if (corr)
     hipLaunchKernelGGL(k_corr, dim3(cdiv((long)M * N, 256)), dim3(256), 0, c->stream, C, M, N, ldc,
@@ -678,24 +450,23 @@ int gemm_nn_p(Ctx* c, int M, int N, int K, double alpha, const double* A, int ld
     }
   }
 
+  lt_mark(c, c->lt_gemm_id, false);
+  if (!use_big(M, N)) {
+    const int rc = gs_gemm_nn(c, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, PREC_FP32);
+    lt_mark(c, c->lt_gemm_id, true);
+    return rc;
+  }
   if (beta != 1.0)
     hipLaunchKernelGGL(k_scale, dim3(cdiv((long)M * N, 256)), dim3(256), 0, c->stream, C, M, N,
                        ldc, beta);
-  lt_mark(c, c->lt_gemm_id, false);
-  if (use_big(M, N)) {
-    launch_big_nn<float>(c, M, N, K, alpha, A, lda, B, ldb, C, ldc);
-  } else {
-    dim3 grid(cdiv(M, BM), cdiv(N, BN), 1);
-    hipLaunchKernelGGL((k_gemm_f32<false, false>), grid, dim3(256), 0, c->stream, M, N, K, K,
-                       alpha, A, lda, B, ldb, C, ldc);
-  }
+  launch_big_nn<float>(c, M, N, K, alpha, A, lda, B, ldb, C, ldc);
   lt_mark(c, c->lt_gemm_id, true);
   QX_CHECK(hipGetLastError());
   return 0;
 }
 
 // FP64 contractions: our 128 x 128 MFMA kernels (mfma_gemm.hip) for sizable
-// outputs, 64 x 64 tiles and matrix-vector kernels for skinny ones
+// outputs, gemm_small.hip and matrix-vector kernels for others
 int gemm_tn(Ctx* c, int M, int N, int K, double alpha, const double* A, int lda, const double* B,
             int ldb, double beta, double* C, int ldc, int corr) {
   if (!use_big(M, N)) return gemm_tn_small(c, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, corr);
@@ -743,14 +514,26 @@ int kb_apply(Ctx* c, const double* psi, double* out, int nb, int, double* slmir_
     explicit TimeGemms(Ctx* cc) : c(cc) { c->lt_gemm_id = 0; }
     ~TimeGemms() { c->lt_gemm_id = -1; }
   } tg(c);
-  int rc = gemm_tn_p(c, c->npj, nb, c->nplwex, 2.0, c->d_B, c->nplwex, psi, c->nplwex, 0.0,
-                     c->d_P, c->npj, 2, prec);
+  int rc;
+  // the small kernels scale the rows by D themselves, unless slmir is wanted
+  const bool fused = !slmir_out && !use_big(c->npj, nb) &&
+                     (prec == PREC_FP32 || !gemv_shape(c->npj, nb));
+  if (fused) {
+    lt_mark(c, c->lt_gemm_id, false);
+    rc = gs_gemm_tn(c, c->npj, nb, c->nplwex, 2.0, c->d_B, c->nplwex, psi, c->nplwex, 0.0, c->d_P,
+                    c->npj, 2, prec, c->d_D);
+    lt_mark(c, c->lt_gemm_id, true);
+  } else {
+    rc = gemm_tn_p(c, c->npj, nb, c->nplwex, 2.0, c->d_B, c->nplwex, psi, c->nplwex, 0.0, c->d_P,
+                   c->npj, 2, prec);
+  }
   if (rc) return rc;
   if (slmir_out)
     QX_CHECK(hipMemcpyAsync(slmir_out, c->d_P, sizeof(double) * (size_t)c->npj * nb,
                             hipMemcpyDeviceToDevice, c->stream));
-  hipLaunchKernelGGL(k_scale_proj, dim3(cdiv((long)c->npj * nb, 256)), dim3(256), 0, c->stream,
-                     c->d_P, c->d_D, c->npj, nb);
+  if (!fused)
+    hipLaunchKernelGGL(k_scale_proj, dim3(cdiv((long)c->npj * nb, 256)), dim3(256), 0, c->stream,
+                       c->d_P, c->d_D, c->npj, nb);
   return gemm_nn_p(c, c->nplwex, nb, c->npj, 1.0, c->d_B, c->nplwex, c->d_P, c->npj, 1.0, out,
                    c->nplwex, prec);
 }
