@@ -20,13 +20,18 @@
 // doubles with a common stride npw_max (the largest sphere) and zeros beyond
 // npw_k, so every stage addresses all k-points by one (k, band) index.
 //
-// Local part, three kernels over all (k, band) blocks of a batch:
+// Local part, three kernels over all (k, band) blocks of a batch: inverse z on
+// the columns of the sphere, per z plane inverse y (on the h range of the
+// sphere) and x, x V(r), forward x and y, and forward z with the kinetic term.
+// T holds only the columns of each sphere ([kb][z][column]), in place.  The
+// two-step transforms of pencil_fast.h take the grids they cover (64 k-points
+// x 20 bands on 30^3, with the nonlocal part: 3.41 -> 0.38 ms); the others run here, on Stockham lines in
+// LDS over dense planes:
 //   k_kzinv  : the column points -> z lines in LDS, inverse FFT along z  -> T
 //   k_kplane : per z plane, the columns into a dense plane in LDS, inverse y
 //              and x, x V(r), forward x and y, back to the columns        -> T
 //   k_kzfwd  : forward z, x 1/N at the sphere points, + |k+G|^2 c (the
 //              kinetic term of ekinetic at k+G); zeros the padding tail.
-// T holds only the columns of each sphere ([kb][z][column]), in place.
 //
 // Nonlocal part: two real products per k-point on the stacked table
 // A_k = [beta_k ; i beta_k] (2 npj rows of 2 npw_max interleaved reals):
@@ -41,7 +46,7 @@
 #include <tuple>
 #include <vector>
 #include <rocsolver/rocsolver.h>
-#include "context.h"
+#include "pencil_fast.h"
 
 namespace qx {
 
@@ -315,6 +320,10 @@ struct KPoints {
   std::vector<std::vector<double>> kin;    // per k: |k+G|^2
   int *d_npw = nullptr, *d_ncol = nullptr, *d_col_p0 = nullptr, *d_col_xy = nullptr,
       *d_pt_z = nullptr;
+  // for the two-step transforms: h range, h and y of the columns, column of a point
+  int *d_hmin = nullptr, *d_hmax = nullptr, *d_col_h = nullptr, *d_col_y = nullptr,
+      *d_pt_col = nullptr;
+  int nH = 1;                              // widest h range
   double* d_kin = nullptr;
   static constexpr int kSlots = 4;
   double* d_slot[kSlots] = {};
@@ -341,6 +350,7 @@ namespace {
 
 void kp_free(KPoints* k) {
   void* ptrs[] = {k->d_npw, k->d_ncol, k->d_col_p0, k->d_col_xy, k->d_pt_z, k->d_kin,
+                  k->d_hmin, k->d_hmax, k->d_col_h, k->d_col_y, k->d_pt_col,
                   k->d_T, k->d_A, k->d_D, k->d_P, k->d_Z, k->d_HZ, k->d_G, k->d_Hs, k->d_Ss,
                   k->d_w, k->d_E, k->d_info, k->d_Cs, k->d_ekin, k->d_lam};
   for (void* p : ptrs)
@@ -471,11 +481,18 @@ int kp_set(Ctx* c, int nk, const double* kfrac, const double* bvec, double ecut,
   }
   const int pm = k->npw_max, cm = k->ncol_max;
   std::vector<int> col_p0((size_t)nk * (cm + 1), 0), col_xy((size_t)nk * cm, 0),
-      pt_z((size_t)nk * pm, 0);
+      pt_z((size_t)nk * pm, 0), col_h((size_t)nk * cm, 0), col_y((size_t)nk * cm, 0),
+      pt_col((size_t)nk * pm, 0), hmin(nk, 0), hmax(nk, 0);
   std::vector<double> kin((size_t)nk * pm, 0.0);
   for (int i = 0; i < nk; ++i) {
     const auto& g = k->hkl[i];
     int col = -1, ph = 0, pk = 0;
+    if (k->npw[i] > 0) hmin[i] = hmax[i] = g[0];
+    for (int p = 0; p < k->npw[i]; ++p) {
+      hmin[i] = std::min(hmin[i], g[3 * p]);
+      hmax[i] = std::max(hmax[i], g[3 * p]);
+    }
+    k->nH = std::max(k->nH, hmax[i] - hmin[i] + 1);
     for (int p = 0; p < k->npw[i]; ++p) {
       const int h = g[3 * p], kk = g[3 * p + 1], l = g[3 * p + 2];
       if (col < 0 || h != ph || kk != pk) {
@@ -483,9 +500,12 @@ int kp_set(Ctx* c, int nk, const double* kfrac, const double* bvec, double ecut,
         col_p0[(size_t)i * (cm + 1) + col] = p;
         col_xy[(size_t)i * cm + col] = ((h % c->n1 + c->n1) % c->n1) +
                                        c->n1 * ((kk % c->n2 + c->n2) % c->n2);
+        col_h[(size_t)i * cm + col] = h - hmin[i];
+        col_y[(size_t)i * cm + col] = (kk % c->n2 + c->n2) % c->n2;
         ph = h;
         pk = kk;
       }
+      pt_col[(size_t)i * pm + p] = col;
       pt_z[(size_t)i * pm + p] = (l % c->n3 + c->n3) % c->n3;
       kin[(size_t)i * pm + p] = k->kin[i][p];
     }
@@ -502,6 +522,11 @@ int kp_set(Ctx* c, int nk, const double* kfrac, const double* bvec, double ecut,
   if (int rc = up(&k->d_col_xy, col_xy)) return rc;
   if (int rc = up(&k->d_pt_z, pt_z)) return rc;
   if (int rc = up(&k->d_kin, kin)) return rc;
+  if (int rc = up(&k->d_hmin, hmin)) return rc;
+  if (int rc = up(&k->d_hmax, hmax)) return rc;
+  if (int rc = up(&k->d_col_h, col_h)) return rc;
+  if (int rc = up(&k->d_col_y, col_y)) return rc;
+  if (int rc = up(&k->d_pt_col, pt_col)) return rc;
   const size_t vbytes = sizeof(double) * 2 * (size_t)pm * nb * nk;
   for (auto*& s : k->d_slot) {
     QX_CHECK(hipMalloc(&s, vbytes));
@@ -600,6 +625,14 @@ int kp_set_kb(Ctx* c, int ik, int npj, const double* beta, const double* D) {
 // band b of k-point k is row k rpk + r0 + b of src and dst
 static int kp_local_run(Ctx* c, KPoints* k, const double* src, double* dst, int kb0, int nkb,
                         int rpk, int r0) {
+  KFastArgs fa{};
+  fa.nb = k->nb; fa.npw_max = k->npw_max; fa.ncol_max = k->ncol_max; fa.kb0 = kb0;
+  fa.rpk = rpk; fa.r0 = r0;
+  fa.npw = k->d_npw; fa.ncol = k->d_ncol; fa.hmin = k->d_hmin; fa.hmax = k->d_hmax;
+  fa.col_p0 = k->d_col_p0; fa.col_h = k->d_col_h; fa.col_y = k->d_col_y;
+  fa.pt_z = k->d_pt_z; fa.pt_col = k->d_pt_col; fa.kin = k->d_kin;
+  const int rf = kp_local_fast(c, fa, k->nH, src, dst, k->d_T, nkb);
+  if (rf != -3) return rf;  // -3: an edge or its LDS is not covered
   const KArgs a = kargs(c, k, kb0, rpk, r0);
   const dim3 gz(cdivu(k->ncol_max, kKCols), nkb);
   hipLaunchKernelGGL(k_kzinv, gz, dim3(kKThreads), 0, c->stream, a, src, k->d_T);

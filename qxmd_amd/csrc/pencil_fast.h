@@ -59,7 +59,7 @@ __host__ __device__ constexpr int zpairs(int N, int elem_bytes) {
 __host__ __device__ inline int slot_phys(int s, int NA, int NB) { return s / NB + NA * (s % NB); }
 
 struct FastArgs {
-  int n1, n2, n3, nH, hmax, npair, ncol, nplwex, nb, bp0;
+  int n1, n2, n3, nH, hmin, hmax, npair, ncol, nplwex, nb, bp0;
   int ya, yb;  // radices of the y edge, n2 = ya * yb
   int sa, sr;  // row strides (elements) of the plane kernel's sphere tile and x strips
   const int *pt_col, *pt_z, *pair_p0, *col_hi, *col_kmod;
@@ -219,18 +219,19 @@ __global__ void __launch_bounds__(kFastThreads) k_zinv_f(FastArgs a, const doubl
 
 // ---- plane: y inverse, x inverse, x V, x forward, y forward ----------------
 // Row offsets in the sphere tile of the natural-x inputs b + NB a of x step A
-// (lane b): row h + hmax for |h| <= hmax, else row 2 hmax + 1, which is kept
-// zero, so every lane loads unconditionally; bit a of *inside is set for the
-// slots inside the sphere, the ones step A' writes back.
+// (lane b): row h - hmin for hmin <= h <= hmax, else row hmax - hmin + 1, which
+// is kept zero, so every lane loads unconditionally; bit a of *inside is set for
+// the slots inside the sphere, the ones step A' writes back.
 template <int NA, int NB>
-__device__ inline void x_offsets(int b, int hmax, int sa, int (&off)[NA], unsigned* inside) {
+__device__ inline void x_offsets(int b, int hmin, int hmax, int sa, int (&off)[NA],
+                                 unsigned* inside) {
   constexpr int N = NA * NB;
   unsigned m = 0;
 #pragma unroll
   for (int a = 0; a < NA; ++a) {
     const int n = b + NB * a;
-    const bool lo = n <= hmax, hi = n >= N - hmax;
-    off[a] = (lo ? n + hmax : (hi ? n - N + hmax : 2 * hmax + 1)) * sa;
+    const bool lo = n >= hmin && n <= hmax, hi = n - N >= hmin && n - N <= hmax;
+    off[a] = (lo ? n - hmin : (hi ? n - N - hmin : hmax - hmin + 1)) * sa;
     m |= (lo || hi) ? 1u << a : 0u;
   }
   *inside = m;
@@ -358,10 +359,10 @@ __device__ inline void y_forward(cplx<T>* A, const FastArgs& a, const cplx<T>* t
 // transformed.  LDS bank conflicts are kept down by the row strides a.sa (sphere
 // tile) and a.sr (x strips), chosen on the host, and by lane maps that put the
 // line (y pass) or row (x pass) index fastest across lanes.
+// in, out: the columns of the plane (they may be the same ones).
 template <typename T, int NA, int NB, int YK>
-__global__ void __launch_bounds__(kPlaneMaxThreads) k_plane_f(FastArgs a, const T* __restrict__ Vp,
-                                                            const cplx<T>* __restrict__ t1,
-                                                            cplx<T>* __restrict__ t2) {
+__device__ inline void plane_body(const FastArgs& a, const T* __restrict__ Vp, int zs,
+                                  const cplx<T>* in, cplx<T>* out) {
   constexpr int N = NA * NB;  // the x edge
   constexpr int RW = plane_rows_per_wave(NA, NB);
   const int n2 = YK == Y_CUBE ? N : a.n2;
@@ -373,14 +374,13 @@ __global__ void __launch_bounds__(kPlaneMaxThreads) k_plane_f(FastArgs a, const 
   cplx<T>* twy = YK == Y_CUBE ? tw : tw + N;
   cplx<T>* A = twy + n2;                             // [nH + 1][sa], y in slot order
   cplx<T>* Rw = A + (nH + 1) * sa + wave * RW * sr;  // this wave's [RW][sr] strip
-  const int zs = blockIdx.x, bp = blockIdx.y;
 
   // lane roles of the x pass (row fastest)
   const int rx = lane % RW, jx = lane / RW;
   const bool actA = jx < NB, actB = jx < NA;
   int xoff[NA];
   unsigned xin;
-  x_offsets<NA, NB>(min(jx, NB - 1), a.hmax, sa, xoff, &xin);
+  x_offsets<NA, NB>(min(jx, NB - 1), a.hmin, a.hmax, sa, xoff, &xin);
   // V(r) row pieces of step B; rows past the grid and idle lanes load a valid
   // row that is not used
   const T* Vz = Vp + (size_t)zs * n2 * N + NB * min(jx, NA - 1);
@@ -393,7 +393,6 @@ __global__ void __launch_bounds__(kPlaneMaxThreads) k_plane_f(FastArgs a, const 
 
   // sphere columns of this plane: loads issued before the LDS fill (real and
   // imaginary parts apart: an array of FP64 pairs went through scratch memory)
-  const cplx<T>* in = t1 + ((size_t)bp * (YK == Y_CUBE ? N : a.n3) + zs) * a.ncol;
   T cr[kPlaneLoads], cim[kPlaneLoads];
   int ci[kPlaneLoads];
 #pragma unroll
@@ -453,9 +452,17 @@ __global__ void __launch_bounds__(kPlaneMaxThreads) k_plane_f(FastArgs a, const 
   }
   __syncthreads();
   y_forward<T, YK, NA, NB>(A, a, twy);
-  cplx<T>* out = t2 + ((size_t)bp * (YK == Y_CUBE ? N : a.n3) + zs) * a.ncol;
   for (int cl = threadIdx.x; cl < a.ncol; cl += blockDim.x)
     out[cl] = A[a.col_hi[cl] * sa + a.col_kmod[cl]];
+}
+
+template <typename T, int NA, int NB, int YK>
+__global__ void __launch_bounds__(kPlaneMaxThreads) k_plane_f(FastArgs a, const T* __restrict__ Vp,
+                                                            const cplx<T>* __restrict__ t1,
+                                                            cplx<T>* __restrict__ t2) {
+  const size_t row =
+      ((size_t)blockIdx.y * (YK == Y_CUBE ? NA * NB : a.n3) + blockIdx.x) * a.ncol;
+  plane_body<T, NA, NB, YK>(a, Vp, blockIdx.x, t1 + row, t2 + row);
 }
 
 // ---- z forward: T2 -> split bands, x1/N, + |G|^2 psi --------------------
@@ -556,7 +563,7 @@ __global__ void __launch_bounds__(rho_max_threads(RG)) k_plane_rho_f(FastArgs a,
   const bool actA = jx < NB, actB = jx < NA;
   int xoff[NA];
   unsigned xin;
-  x_offsets<NA, NB>(min(jx, NB - 1), a.hmax, sa, xoff, &xin);
+  x_offsets<NA, NB>(min(jx, NB - 1), a.hmin, a.hmax, sa, xoff, &xin);
   load_tw<T>(tw, a.tw, N);
   if constexpr (YK != Y_CUBE) load_tw<T>(twy, a.tw + 2 * N, n2);
   __syncthreads();
@@ -616,6 +623,111 @@ __global__ void __launch_bounds__(rho_max_threads(RG)) k_plane_rho_f(FastArgs a,
   }
 }
 
+// ---- Bloch bands (kpoint.hip): one complex band per transform, a sphere per
+// k-point, the columns of a (k, band) block transformed in place ----------------
+struct KFastArgs {
+  FastArgs f;          // grid, y radices, strides, twiddles
+  int nb, npw_max, ncol_max, kb0;
+  int rpk, r0;         // band rows of a k-point in the src/dst arrays, first row used
+  const int *npw, *ncol, *hmin, *hmax;  // [k]
+  const int* col_p0;   // [k][ncol_max + 1]: first point of column c
+  const int *col_h, *col_y;             // [k][ncol_max]: h, y index of column c
+  const int *pt_z, *pt_col;             // [k][npw_max]
+  const double* kin;   // [k][npw_max]: |k+G|^2
+};
+constexpr int kKFastCols = 16;  // columns per block of the z kernels
+
+template <int NA, int NB>
+__global__ void __launch_bounds__(kFastThreads)
+    k_kzinv_f(KFastArgs a, const double* __restrict__ psi, cplx<double>* __restrict__ T) {
+  constexpr int N = NA * NB;
+  __shared__ cplx<double> tw[N], lines[kKFastCols][N];
+  const int kb = a.kb0 + (int)blockIdx.y, k = kb / a.nb;
+  const int nc = a.ncol[k], c0 = (int)blockIdx.x * kKFastCols;
+  if (c0 >= nc) return;
+  const int cn = min(kKFastCols, nc - c0);
+  load_tw<double>(tw, a.f.tw + 2 * (a.f.n1 + a.f.n2), N);
+  for (int i = threadIdx.x; i < cn * N; i += blockDim.x) lines[i / N][i % N] = mk<double>(0.0, 0.0);
+  __syncthreads();
+  const int* cp = a.col_p0 + (size_t)k * (a.ncol_max + 1);
+  const int *pz = a.pt_z + (size_t)k * a.npw_max, *pc = a.pt_col + (size_t)k * a.npw_max;
+  const double2* src = reinterpret_cast<const double2*>(
+      psi + ((size_t)k * a.rpk + a.r0 + (kb - k * a.nb)) * 2 * a.npw_max);
+  const int p1 = cp[c0 + cn];
+  for (int p = cp[c0] + (int)threadIdx.x; p < p1; p += blockDim.x) {
+    const double2 v = src[p];
+    lines[pc[p] - c0][pz[p]] = mk<double>(v.x, v.y);
+  }
+  __syncthreads();
+  for (int it = threadIdx.x; it < cn * NB; it += blockDim.x)
+    np_stepA<double, NA>(lines[it / NB], it % NB, NB, tw, +1);
+  __syncthreads();
+  for (int it = threadIdx.x; it < cn * NA; it += blockDim.x)
+    np_stepB<double, NB>(lines[it / NA], it % NA, +1);
+  __syncthreads();
+  cplx<double>* out = T + (size_t)blockIdx.y * N * a.ncol_max + c0;
+  for (int i = threadIdx.x; i < kKFastCols * N; i += blockDim.x) {
+    const int zs = i / kKFastCols, cl = i % kKFastCols;
+    if (cl < cn) out[(size_t)zs * a.ncol_max + cl] = lines[cl][zs];
+  }
+}
+
+template <int NA, int NB, int YK>
+__global__ void __launch_bounds__(kPlaneMaxThreads)
+    k_kplane_f(KFastArgs a, const double* __restrict__ Vp, cplx<double>* T) {
+  const int k = (a.kb0 + (int)blockIdx.y) / a.nb;
+  FastArgs f = a.f;
+  f.ncol = a.ncol[k];
+  f.hmin = a.hmin[k];
+  f.hmax = a.hmax[k];
+  f.nH = f.hmax - f.hmin + 1;
+  f.col_hi = a.col_h + (size_t)k * a.ncol_max;
+  f.col_kmod = a.col_y + (size_t)k * a.ncol_max;
+  cplx<double>* row =
+      T + ((size_t)blockIdx.y * (YK == Y_CUBE ? NA * NB : f.n3) + blockIdx.x) * a.ncol_max;
+  plane_body<double, NA, NB, YK>(f, Vp, blockIdx.x, row, row);
+}
+
+template <int NA, int NB>
+__global__ void __launch_bounds__(kFastThreads)
+    k_kzfwd_f(KFastArgs a, const double* __restrict__ psi, const cplx<double>* __restrict__ T,
+              double* __restrict__ out, double scale) {
+  constexpr int N = NA * NB;
+  __shared__ cplx<double> tw[N], lines[kKFastCols][N];
+  const int kb = a.kb0 + (int)blockIdx.y, k = kb / a.nb;
+  const int nc = a.ncol[k], np = a.npw[k];
+  const size_t row = ((size_t)k * a.rpk + a.r0 + (kb - k * a.nb)) * 2 * a.npw_max;
+  if (blockIdx.x == 0)  // the padding beyond npw_k stays zero
+    for (int i = 2 * np + (int)threadIdx.x; i < 2 * a.npw_max; i += blockDim.x) out[row + i] = 0.0;
+  const int c0 = (int)blockIdx.x * kKFastCols;
+  if (c0 >= nc) return;
+  const int cn = min(kKFastCols, nc - c0);
+  load_tw<double>(tw, a.f.tw + 2 * (a.f.n1 + a.f.n2), N);
+  const cplx<double>* in = T + (size_t)blockIdx.y * N * a.ncol_max + c0;
+  for (int i = threadIdx.x; i < kKFastCols * N; i += blockDim.x) {
+    const int zs = i / kKFastCols, cl = i % kKFastCols;
+    if (cl < cn) lines[cl][zs] = in[(size_t)zs * a.ncol_max + cl];
+  }
+  __syncthreads();
+  for (int it = threadIdx.x; it < cn * NA; it += blockDim.x)
+    pn_stepB<double, NB>(lines[it / NA], it % NA, tw, -1);
+  __syncthreads();
+  for (int it = threadIdx.x; it < cn * NB; it += blockDim.x)
+    pn_stepA<double, NA>(lines[it / NB], it % NB, NB, -1);
+  __syncthreads();
+  const int* cp = a.col_p0 + (size_t)k * (a.ncol_max + 1);
+  const int *pz = a.pt_z + (size_t)k * a.npw_max, *pc = a.pt_col + (size_t)k * a.npw_max;
+  const double* kin = a.kin + (size_t)k * a.npw_max;
+  const double2* src = reinterpret_cast<const double2*>(psi + row);
+  double2* dst = reinterpret_cast<double2*>(out + row);
+  const int p1 = cp[c0 + cn];
+  for (int p = cp[c0] + (int)threadIdx.x; p < p1; p += blockDim.x) {
+    const cplx<double> v = lines[pc[p] - c0][pz[p]];
+    const double2 c = src[p];
+    dst[p] = make_double2(v.x * scale + kin[p] * c.x, v.y * scale + kin[p] * c.y);
+  }
+}
+
 // ---- launch table: the kernels of one edge and precision ---------------------
 constexpr int kRhoKinds = 3;  // row groups per wavefront of the density kernel: 2, 4, 6
 template <typename T>
@@ -629,6 +741,10 @@ struct EdgeKernels {
   ZFwd zfwd = nullptr;
   Plane plane[3] = {};            // x edge; by YKind
   Rho rho[3][kRhoKinds] = {};     // 6 row groups for cubes only
+  // Bloch bands (FP64 only)
+  void (*kzinv)(KFastArgs, const double*, cplx<double>*) = nullptr;
+  void (*kzfwd)(KFastArgs, const double*, const cplx<double>*, double*, double) = nullptr;
+  void (*kplane[3])(KFastArgs, const double*, cplx<double>*) = {};
 };
 template <typename T>
 using EdgeLookup = bool (*)(int n, EdgeKernels<T>* k);
@@ -639,5 +755,10 @@ using EdgeLookup = bool (*)(int n, EdgeKernels<T>* k);
 QX_DECL_GROUP(0) QX_DECL_GROUP(1) QX_DECL_GROUP(2) QX_DECL_GROUP(3)
 QX_DECL_GROUP(4) QX_DECL_GROUP(5) QX_DECL_GROUP(6) QX_DECL_GROUP(7)
 #undef QX_DECL_GROUP
+
+// Bloch-band local part: launches zinv, plane, zfwd for nkb blocks of T; -3 when
+// the grid or its LDS is not covered.  nH: the widest sphere's h extent.
+int kp_local_fast(Ctx* c, KFastArgs a, int nH, const double* src, double* dst, double2* T,
+                  int nkb);
 
 }  // namespace qx

@@ -128,6 +128,7 @@ static FastArgs fast_args(Ctx* c, const PlaneShape& s, int nb, int bp0) {
   a.ya = s.ya; a.yb = s.yb;
   a.nH = c->pc.nH;
   a.hmax = (c->pc.nH - 1) / 2;
+  a.hmin = -a.hmax;
   a.npair = c->pc.npair;
   a.ncol = c->pc.ncol;
   a.nplwex = c->nplwex;
@@ -446,6 +447,35 @@ static int local_fast_t(Ctx* c, const double* psi, double* out, int nb, int accu
                        accumulate, 1.0 / (double)c->N, mid ? mid->kb32 : nullptr);
     lt_mark(c, 1, true);
   }
+  QX_CHECK(hipGetLastError());
+  return 0;
+}
+
+int kp_local_fast(Ctx* c, KFastArgs a, int nH, const double* src, double* dst, double2* T,
+                  int nkb) {
+  if (!fast_ok(c) || !c->d_Vp || nH > c->n1) return -3;
+  PlaneShape s = plane_shape<double>(c);
+  s.nH = nH;
+  const EdgeKernels<double> kz = edge_kernels<double>(c->n3);
+  const auto plane = edge_kernels<double>(c->n1).kplane[s.yk];
+  if (!kz.kzinv || !kz.kzfwd || !plane) return -3;
+  // as many wavefronts as the x pass has row groups for, 4 or 8 (small cells:
+  // 30 x 30 planes have three groups of ten rows)
+  int nwave = plane_waves(s);
+  if (nwave == 8 && (s.n2 + s.rw - 1) / s.rw <= 4) nwave = 4;
+  if (nwave < 1) return -3;
+  FastArgs f = fast_args(c, s, 0, 0);
+  plane_strides(s, nwave, &f.sa, &f.sr);
+  const size_t lp = s.lds(f.sa, f.sr, nwave);
+  if (lp > kCuLds) return -3;
+  plane_lds_optin(reinterpret_cast<const void*>(plane), lp);
+  a.f = f;
+  cplx<double>* t = reinterpret_cast<cplx<double>*>(T);
+  const dim3 gz((unsigned)((a.ncol_max + kKFastCols - 1) / kKFastCols), nkb);
+  hipLaunchKernelGGL(kz.kzinv, gz, dim3(kFastThreads), 0, c->stream, a, src, t);
+  hipLaunchKernelGGL(plane, dim3(c->n3, nkb), dim3(64 * nwave), lp, c->stream, a, c->d_Vp, t);
+  hipLaunchKernelGGL(kz.kzfwd, gz, dim3(kFastThreads), 0, c->stream, a, src, t, dst,
+                     1.0 / (double)c->N);
   QX_CHECK(hipGetLastError());
   return 0;
 }

@@ -21,6 +21,13 @@ static void fill(EdgeKernels<T>* k) {
   k->rho[Y_R10][1] = k_plane_rho_f<T, NA, NB, Y_R10, 4>;
   k->rho[Y_R16][0] = k_plane_rho_f<T, NA, NB, Y_R16, 2>;
   k->rho[Y_R16][1] = k_plane_rho_f<T, NA, NB, Y_R16, 4>;
+  if constexpr (sizeof(T) == 8) {
+    k->kzinv = k_kzinv_f<NA, NB>;
+    k->kzfwd = k_kzfwd_f<NA, NB>;
+    k->kplane[Y_CUBE] = k_kplane_f<NA, NB, Y_CUBE>;
+    k->kplane[Y_R10] = k_kplane_f<NA, NB, Y_R10>;
+    k->kplane[Y_R16] = k_kplane_f<NA, NB, Y_R16>;
+  }
 }
 
 template <typename T>
