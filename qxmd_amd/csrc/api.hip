@@ -332,7 +332,7 @@ int qx_destroy(qx_ctx* h) {
   void* ptrs[] = {c->d_perm, c->d_pt_col, c->d_pt_z, c->d_pair_p0, c->d_col_hi, c->d_col_kmod,
                   c->d_kin, c->d_tw, c->d_V, c->d_Vf, c->d_Vp, c->d_Vpf, c->d_B, c->d_D, c->d_t1, c->d_t2, c->d_P,
                   c->d_small, c->d_rho_part, c->d_rho, c->d_scal, c->d_sync, c->d_dwork, c->d_bb,
-                  c->d_gs};
+                  c->d_gs, c->d_frc};
   for (void* p : ptrs)
     if (p) (void)hipFree(p);
   if (c->h_flag) (void)hipHostFree(c->h_flag);

@@ -85,6 +85,8 @@ struct Ctx {
   double *d_scal = nullptr;               // scalar work (device)
   int* d_sync = nullptr;                  // grid-barrier counter and error flags
   double* d_dwork = nullptr;              // dense eigensolver work (8 nbmax^2 + ...)
+  double* d_frc = nullptr;                // workspace of the nonlocal forces
+  size_t frc_len = 0;
   double* d_gs = nullptr;                 // K-slice partials of the small products
   size_t gs_len = 0;
   double* d_bb = nullptr;                 // band-by-band CG: scalars, then chunk sums
