@@ -160,7 +160,9 @@ int schmidt_dev(Ctx* c, double* psi, int nb, int* ok_host, int prec, bool split_
   // psi'_ib = sum_jb Linv(ib,jb) psi_jb: gemm_nn's B[n*ldb + k] = Linv(n,k)
   if (split) return band_nn(c, nb, 1.0, ps, Linv, nb, 0.0, psi);  // reads the split planes
   double* out = c->d_slot[5];
-  if ((rc = gemm_nn_p(c, n, nb, nb, 1.0, psi, n, Linv, nb, 0.0, out, n, prec))) return rc;
+  if ((rc = gemm_nn_p(c, n, nb, nb, 1.0, psi, n, Linv, nb, 0.0, out, n, prec,
+                      true)))
+    return rc;
   QX_CHECK(hipMemcpyAsync(psi, out, sizeof(double) * (size_t)n * nb, hipMemcpyDeviceToDevice,
                           c->stream));
   return 0;

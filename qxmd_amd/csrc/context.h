@@ -253,7 +253,7 @@ int cg_graph_entries(Ctx* c);
 int mg_dgemm_tn(Ctx* c, int M, int N, int K, double alpha, const double* A, int lda,
                 const double* B, int ldb, double beta, double* C, int ldc, int corr);
 int mg_dgemm_nn(Ctx* c, int M, int N, int K, double alpha, const double* A, int lda,
-                const double* B, int ldb, double beta, double* C, int ldc);
+                const double* B, int ldb, double beta, double* C, int ldc, bool upper = false);
 template <typename T, typename TC>
 int mg_bf3_tn(Ctx* c, int M, int N, int K, double alpha, const T* A, int lda, const T* B, int ldb,
               double beta, TC* C, int ldc, int corr);
@@ -388,7 +388,7 @@ int tridiag_wg(Ctx* c, double* a, int n, double* d, double* e);
 int gemm_tn(Ctx* c, int M, int N, int K, double alpha, const double* A, int lda, const double* B,
             int ldb, double beta, double* C, int ldc, int corr);
 int gemm_nn(Ctx* c, int M, int N, int K, double alpha, const double* A, int lda, const double* B,
-            int ldb, double beta, double* C, int ldc);
+            int ldb, double beta, double* C, int ldc, bool upper = false);
 // the products with a dimension of the output below 256 (gemm_small.hip), in
 // either precision, over `batch` operands at the given strides; rscale: a
 // factor per row m of C (TN)
@@ -404,6 +404,7 @@ int gs_gemm_nn(Ctx* c, int M, int N, int K, double alpha, const double* A, int l
 int gemm_tn_p(Ctx* c, int M, int N, int K, double alpha, const double* A, int lda,
               const double* B, int ldb, double beta, double* C, int ldc, int corr, int prec);
 int gemm_nn_p(Ctx* c, int M, int N, int K, double alpha, const double* A, int lda,
-              const double* B, int ldb, double beta, double* C, int ldc, int prec);
+              const double* B, int ldb, double beta, double* C, int ldc, int prec,
+              bool upper = false);
 
 }  // namespace qx

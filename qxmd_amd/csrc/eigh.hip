@@ -896,7 +896,7 @@ static int chol_qr(Ctx* c, double* z, int n, double* gram, double* linv, double*
     if (shifted && pass == 0)
       hipLaunchKernelGGL(k_add_diag, dim3((n + 255) / 256), dim3(256), 0, c->stream, gram, n, shift);
     if ((rc = dense_chol_inv(c, gram, n, linv, ok + 2 * pass, ok + 7))) return rc;
-    if ((rc = gemm_nn(c, n, n, n, 1.0, z, n, linv, n, 0.0, tmp, n))) return rc;
+    if ((rc = gemm_nn(c, n, n, n, 1.0, z, n, linv, n, 0.0, tmp, n, true))) return rc;
     QX_CHECK(hipMemcpyAsync(z, tmp, sizeof(double) * (size_t)n * n, hipMemcpyDeviceToDevice,
                             c->stream));
   }

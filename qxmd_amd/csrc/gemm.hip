@@ -438,8 +438,8 @@ int gemm_tn_p(Ctx* c, int M, int N, int K, double alpha, const double* A, int ld
 }
 
 int gemm_nn_p(Ctx* c, int M, int N, int K, double alpha, const double* A, int lda, const double* B,
-              int ldb, double beta, double* C, int ldc, int prec) {
-  if (prec != PREC_FP32) return gemm_nn(c, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc);
+              int ldb, double beta, double* C, int ldc, int prec, bool upper) {
+  if (prec != PREC_FP32) return gemm_nn(c, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, upper);
   if (M <= 0 || N <= 0) return 0;
   if (use_big(M, N)) {
     if (lt_enabled()) {
@@ -484,8 +484,9 @@ int gemm_tn(Ctx* c, int M, int N, int K, double alpha, const double* A, int lda,
   return gemm_tn_small(c, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, corr);
 }
 
+// upper: the caller's B has zeros at B(k, n), k > n, which the large kernels skip
 int gemm_nn(Ctx* c, int M, int N, int K, double alpha, const double* A, int lda, const double* B,
-            int ldb, double beta, double* C, int ldc) {
+            int ldb, double beta, double* C, int ldc, bool upper) {
   if (!use_big(M, N)) return gemm_nn_small(c, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc);
   if (lt_enabled()) {
     if (lt_dgemm(c, false, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc) != 0)
@@ -493,7 +494,7 @@ int gemm_nn(Ctx* c, int M, int N, int K, double alpha, const double* A, int lda,
     QX_CHECK(hipGetLastError());
     return 0;
   }
-  const int rc = mg_dgemm_nn(c, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc);
+  const int rc = mg_dgemm_nn(c, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, upper);
   if (rc != -3) return rc;
   return gemm_nn_small(c, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc);
 }

@@ -9,9 +9,10 @@
 //        psi U (Sources/eigen.f90:1485-1509), psi L^-T (Sources/schmidt.f90:284-313).
 //
 // Tiles: 128 x 128 outputs per 256-thread workgroup, four wavefronts of
-// 64 x 64.  FP64: a 4 x 4 grid of v_mfma_f64_16x16x4f64 blocks per wavefront,
-// K staged 16 at a time through double-buffered LDS (one barrier per stage),
-// the next stage's global loads in flight during the current stage's MFMAs.
+// 64 x 64.  FP64: up to a 4 x 4 grid of v_mfma_f64_16x16x4f64 blocks per
+// wavefront, K staged 16 at a time through double-buffered LDS (one barrier per
+// stage), the next stage's global loads in flight during the current stage's
+// MFMAs.
 //
 // Split bf16x3 (the mixed form's FP32-class products): every FP32 (or FP64)
 // operand x is split while staged into x_hi = bf16(x) and x_lo = bf16(x - x_hi);
@@ -54,7 +55,7 @@ typedef float f4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf8 __attribute__((ext_vector_type(8)));
 
 constexpr int TE = 128;                    // output tile edge
-constexpr int KT64 = 16, LP64 = TE + 4;    // FP64 K stage, LDS row pitch (doubles)
+constexpr int KT64 = 16;                   // FP64 K stage
 constexpr int KT16 = 32, LP16 = KT16 + 8;  // bf16 K stage, LDS row pitch (bf16)
 constexpr int kXcd = 8;                    // XCDs the dispatcher round-robins over
 
@@ -72,6 +73,13 @@ struct Sk {
   int ldc, corr;
   long alo, blo;  // pre-split operands: element offset of the lo half after the hi half
   int tm, tn;     // output tile (TE x TE, or 96 along an edge for the FP64 kernels)
+  int T;          // output tiles
+  // TN with B = A: C is symmetric, the tiles on and below the diagonal are
+  // computed (tm == tn) and written to both sides
+  int sym;
+  // NN with an upper triangular B (B(k, n) = 0 for k > n): a tile worked by one
+  // workgroup ends at the K stage that holds its last column
+  int tri;
 };
 
 // logical workgroup: XCD x = blockIdx % 8 takes the x-th contiguous eighth
@@ -89,10 +97,15 @@ __device__ inline int logical_wg(int G) {
 // share each K stage of both operands in their L2.  Empty for workgroups past
 // the last non-empty slice.
 __device__ inline void sk_range(const Sk& sk, int lb, long& g0, long& g1) {
-  const int T = sk.tiles_m * sk.tiles_n;
+  const int T = sk.T;
   if (sk.S > 0) {
     const int s = lb / T, t = lb - s * T;
-    const int a = s * sk.nks, b = min(sk.nk, a + sk.nks);
+    const int a = s * sk.nks;
+    int b = min(sk.nk, a + sk.nks);
+    if (sk.tri) {  // one slice
+      const int n1 = ((sk.nfast ? t % sk.tiles_n : t / sk.tiles_m) + 1) * sk.tn;
+      b = min(b, (n1 + KT64 - 1) / KT64);
+    }
     if (s >= sk.S || a >= b) {
       g0 = g1 = 0;
       return;
@@ -108,7 +121,13 @@ __device__ inline void sk_range(const Sk& sk, int lb, long& g0, long& g1) {
 // origin of output tile t: M index fastest, or N index fastest (NN products:
 // consecutive tiles share the rows of the long operand A)
 __device__ inline void tile_origin(const Sk& sk, int t, int& m0, int& n0) {
-  if (sk.nfast) {
+  if (sk.sym) {  // t = i (i + 1) / 2 + j, j <= i
+    int i = (int)((sqrtf(8.0f * (float)t + 1.0f) - 1.0f) * 0.5f);
+    while ((i + 1) * (i + 2) / 2 <= t) ++i;
+    while (i * (i + 1) / 2 > t) --i;
+    m0 = i * sk.tm;
+    n0 = (t - i * (i + 1) / 2) * sk.tn;
+  } else if (sk.nfast) {
     m0 = (t / sk.tiles_n) * sk.tm;
     n0 = (t % sk.tiles_n) * sk.tn;
   } else {
@@ -130,26 +149,50 @@ __device__ inline double corr_term(int corr, const T* A, int lda, const T* B, in
 // ---------------------------------------------------------------- FP64 ----
 // Output tile 32 BI x 32 BJ (BI, BJ = 4 or 3: 128 or 96 along each edge, so
 // that 540 bands or 864 projectors waste little of the last tile), four
-// wavefronts of 16 BI x 16 BJ in a 2 x 2 layout.  Operands move in 16-byte
-// chunks: a k-contiguous row of the K stage is 8 chunks (8 threads read 128
-// consecutive bytes), an m-contiguous k row is TM / 2 chunks.
+// wavefronts of 16 BI x 16 BJ in a 2 x 2 layout, three workgroups per CU of the
+// 96 x 96 tile (48 KB LDS, 168 registers), two of the others.  Operands move in
+// 16-byte chunks: a k-contiguous row of the K stage is 8 chunks, an m-contiguous
+// k row TM / 2.
+// The MFMAs bound it (71 TF/s from registers alone on this card), so the LDS
+// traffic beside them has to stay off the critical path:
+// - stage row k keeps column x at x ^ f64_sw(k): the transposing 8-byte stores
+//   of a k-contiguous operand (8 rows x 4 k pairs per half wavefront) and the
+//   fragment reads (16 columns of two consecutive k per half wavefront) both
+//   touch every bank once; padded rows left either with two-way conflicts
+// - the fragments of the next four k are read before the MFMAs of the current
+//   four are issued, and the next stage is stored before the last four's, so a
+//   wavefront waits for LDS only at the start of a stage
+// 864 x 432 x 44640 TN: padded rows, two workgroups per CU 695 us (48 TF/s); the
+// swizzle 655; + stores before the last MFMAs 610; + three workgroups 587.
+// KB products of 540 bands of the 216-atom cell: 1.89 -> 1.53 ms.
+__device__ inline constexpr int f64_sw(int k) {
+  return (8 * ((k >> 1) & 1)) ^ (16 * ((k >> 2) & 1)) ^ (16 * (k & 1));
+}
 template <bool AK, int BI, int BJ>
-__global__ void __launch_bounds__(256, 2)
+__global__ void __launch_bounds__(256, BI == 3 && BJ == 3 ? 3 : 2)
     k_mg_f64(Sk sk, const double* __restrict__ A, int lda, const double* __restrict__ B, int ldb,
              double* __restrict__ C, double* __restrict__ Wp) {
   constexpr int TM = 32 * BI, TN = 32 * BJ;
-  constexpr int LPM = TM + 4, LPN = TN + 4;
   constexpr int CA = TM * KT64 / 2 / 256, CB = TN * KT64 / 2 / 256;  // chunks per thread
   static_assert(TM * KT64 / 2 % 256 == 0 && TN * KT64 / 2 % 256 == 0, "chunk split");
-  __shared__ double As[2][KT64][LPM];
-  __shared__ double Bs[2][KT64][LPN];
+  __shared__ __align__(16) double As[2][KT64][TM];
+  __shared__ __align__(16) double Bs[2][KT64][TN];
   const int M = sk.M, N = sk.N, K = sk.K;
   const int lb = logical_wg(sk.G);
   long g0, g1;
   sk_range(sk, lb, g0, g1);
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = (wave & 1) * (TM / 2), wn = (wave >> 1) * (TN / 2);
   for (long g = g0; g < g1;) {
+    // opaque per segment: the compiler otherwise hoists every address of the
+    // segment out of this loop and spills them (96 x 96: 256 bytes per lane)
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = (wave & 1) * (TM / 2), wn = (wave >> 1) * (TN / 2);
+    // k-contiguous chunk u of this thread: row (4 u + wave) 8 + cr, k pair cj (the
+    // lower half wavefront takes the first four pairs of its 8 rows)
+    const int cj = (lane & 3) | ((lane >> 5) << 2), cr = 8 * wave + ((lane >> 2) & 7);
+    // fragment reads: k of the lane within a step of four, column within 16
+    const int kl = lane >> 4, cc = (lane & 15) ^ (8 * ((kl >> 1) & 1));
     const int t = (int)(g / sk.nk);
     const int s0 = (int)(g - (long)t * sk.nk);
     const int s1 = (int)min((long)sk.nk, g1 - (long)t * sk.nk);
@@ -161,114 +204,146 @@ __global__ void __launch_bounds__(256, 2)
     for (int i = 0; i < BI; ++i)
 #pragma unroll
       for (int j = 0; j < BJ; ++j) acc[i][j] = d4{0.0, 0.0, 0.0, 0.0};
+    // Chunk addresses: 32-bit byte offsets from the tile's (uniform) corner of a
+    // stage.  Columns past N and k-contiguous rows past M read the last row again;
+    // an m-contiguous chunk past M reads the chunk that holds row M - 1 (with an
+    // odd M also the row's padding: lda is even): those outputs are not stored.
     double2 ra[CA], rb[CB];
-    // chunk u of this thread: k-contiguous -> row c / 8, k 2 (c % 8);
-    // m-contiguous -> k row c / (TM / 2), m 2 (c % (TM / 2))
+    unsigned oa[CA], ob[CB];
+#pragma unroll
+    for (int u = 0; u < CA; ++u) {
+      const int c = tid + 256 * u;
+      oa[u] = 8u * (AK ? (unsigned)(min(32 * u + cr, M - 1 - m0) * lda + 2 * cj)
+                       : (unsigned)((c / (TM / 2)) * lda +
+                                    min(2 * (c % (TM / 2)), ((M - 1) & ~1) - m0)));
+    }
+#pragma unroll
+    for (int u = 0; u < CB; ++u)
+      ob[u] = 8u * (unsigned)(min(32 * u + cr, N - 1 - n0) * ldb + 2 * cj);
+    const double* A0 = A + (AK ? (size_t)m0 * lda : (size_t)m0);
+    const double* B0 = B + (size_t)n0 * ldb;
+    auto at = [](const double* p, unsigned o) {
+      return reinterpret_cast<const double*>(reinterpret_cast<const char*>(p) + o);
+    };
     auto fetch = [&](int k0) {
-      const bool full = k0 + KT64 <= ke;
+      const double* Ak = A0 + (AK ? (size_t)k0 : (size_t)k0 * lda);
+#pragma unroll
+      for (int u = 0; u < CA; ++u) ra[u] = *reinterpret_cast<const double2*>(at(Ak, oa[u]));
+#pragma unroll
+      for (int u = 0; u < CB; ++u) rb[u] = *reinterpret_cast<const double2*>(at(B0 + k0, ob[u]));
+    };
+    // the stage that K ends in: zeros past ke, the loads kept before it
+    auto fetch_tail = [&](int k0) {
+      const int d0 = min(0, ke - 1 - (k0 + 2 * cj)), d1 = min(1, ke - 1 - (k0 + 2 * cj));
+      auto pair = [&](const double* p) {
+        const double x = p[d0], y = p[d1];
+        return make_double2(d0 == 0 ? x : 0.0, d1 == 1 ? y : 0.0);
+      };
 #pragma unroll
       for (int u = 0; u < CA; ++u) {
-        const int c = tid + 256 * u;
         if (AK) {
-          const int row = c >> 3, k = k0 + 2 * (c & 7);
-          const double* p = A + (size_t)min(m0 + row, M - 1) * lda + k;
-          if (full) {
-            ra[u] = *reinterpret_cast<const double2*>(p);
-          } else {
-            ra[u].x = k < ke ? p[0] : 0.0;
-            ra[u].y = k + 1 < ke ? p[1] : 0.0;
-          }
+          ra[u] = pair(at(A0 + k0, oa[u]));
         } else {
-          const int kr = c / (TM / 2), m = m0 + 2 * (c % (TM / 2)), k = k0 + kr;
-          const double* p = A + (size_t)min(k, K - 1) * lda + m;
-          if (k < ke && m + 2 <= M) {
-            ra[u] = *reinterpret_cast<const double2*>(p);
-          } else {
-            ra[u].x = (k < ke && m < M) ? p[0] : 0.0;
-            ra[u].y = (k < ke && m + 1 < M) ? p[1] : 0.0;
-          }
+          const int d = min(0, ke - 1 - (k0 + (tid + 256 * u) / (TM / 2)));
+          const double2 v = *reinterpret_cast<const double2*>(
+              at(A0 + (size_t)k0 * lda, oa[u]) + (long)d * lda);
+          ra[u] = d == 0 ? v : make_double2(0.0, 0.0);
         }
       }
 #pragma unroll
-      for (int u = 0; u < CB; ++u) {
-        const int c = tid + 256 * u;
-        const int row = c >> 3, k = k0 + 2 * (c & 7);
-        const double* p = B + (size_t)min(n0 + row, N - 1) * ldb + k;
-        if (full) {
-          rb[u] = *reinterpret_cast<const double2*>(p);
-        } else {
-          rb[u].x = k < ke ? p[0] : 0.0;
-          rb[u].y = k + 1 < ke ? p[1] : 0.0;
-        }
-      }
+      for (int u = 0; u < CB; ++u) rb[u] = pair(at(B0 + k0, ob[u]));
     };
     auto stash = [&](int buf) {
+      const int k = 2 * cj, x0 = f64_sw(k), x1 = f64_sw(k + 1);
 #pragma unroll
       for (int u = 0; u < CA; ++u) {
-        const int c = tid + 256 * u;
         if (AK) {
-          const int row = c >> 3, k = 2 * (c & 7);
-          As[buf][k][row] = ra[u].x;
-          As[buf][k + 1][row] = ra[u].y;
+          As[buf][k][(32 * u + cr) ^ x0] = ra[u].x;
+          As[buf][k + 1][(32 * u + cr) ^ x1] = ra[u].y;
         } else {
+          const int c = tid + 256 * u;
           const int kr = c / (TM / 2), m = 2 * (c % (TM / 2));
-          *reinterpret_cast<double2*>(&As[buf][kr][m]) = ra[u];
+          *reinterpret_cast<double2*>(&As[buf][kr][m ^ f64_sw(kr)]) = ra[u];
         }
       }
 #pragma unroll
       for (int u = 0; u < CB; ++u) {
-        const int c = tid + 256 * u;
-        const int row = c >> 3, k = 2 * (c & 7);
-        Bs[buf][k][row] = rb[u].x;
-        Bs[buf][k + 1][row] = rb[u].y;
+        Bs[buf][k][(32 * u + cr) ^ x0] = rb[u].x;
+        Bs[buf][k + 1][(32 * u + cr) ^ x1] = rb[u].y;
       }
     };
-    int buf = 0;
-    fetch(kb);
-    stash(0);
-    __syncthreads();
-    for (int k0 = kb; k0 < ke; k0 += KT64) {
-      const bool more = k0 + KT64 < ke;
-      if (more) fetch(k0 + KT64);
+    auto frags = [&](int buf, int k4, double(&a)[BI], double(&b)[BJ]) {
+      const int x = (16 * (kl & 1)) ^ (16 * ((k4 >> 2) & 1));
+      const double *ar = &As[buf][k4 + kl][0], *br = &Bs[buf][k4 + kl][0];
 #pragma unroll
-      for (int k4 = 0; k4 < KT64; k4 += 4) {
-        const int kr = k4 + (lane >> 4), c = lane & 15;
-        double a[BI], b[BJ];
+      for (int i = 0; i < BI; ++i) a[i] = ar[((wm + 16 * i) ^ x) + cc];
 #pragma unroll
-        for (int i = 0; i < BI; ++i) a[i] = As[buf][kr][wm + 16 * i + c];
+      for (int j = 0; j < BJ; ++j) b[j] = br[((wn + 16 * j) ^ x) + cc];
+    };
+    // MFMAs of a stage; the next one, if fetched, is stored before the last four k
+    auto compute = [&](int buf, bool more) {
+      double a[2][BI], b[2][BJ];
+      frags(buf, 0, a[0], b[0]);
 #pragma unroll
-        for (int j = 0; j < BJ; ++j) b[j] = Bs[buf][kr][wn + 16 * j + c];
+      for (int q = 0; q < KT64 / 4; ++q) {
+        if (q + 1 < KT64 / 4) frags(buf, 4 * q + 4, a[(q + 1) & 1], b[(q + 1) & 1]);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int i = 0; i < BI; ++i)
 #pragma unroll
           for (int j = 0; j < BJ; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i], b[j], acc[i][j], 0, 0, 0);
+            acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[q & 1][i], b[q & 1][j], acc[i][j],
+                                                             0, 0, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        if (q == KT64 / 4 - 2 && more) stash(buf ^ 1);
       }
-      if (more) stash(buf ^ 1);
       __syncthreads();
-      buf ^= 1;
+    };
+    int buf = 0;
+    const int kf = kb + (ke - kb) / KT64 * KT64;  // end of the full stages
+    if (kf > kb) {
+      fetch(kb);
+      stash(0);
+      __syncthreads();
+      for (int k0 = kb; k0 < kf; k0 += KT64, buf ^= 1) {
+        const bool more = k0 + KT64 < kf;
+        if (more) fetch(k0 + KT64);
+        compute(buf, more);
+      }
+    }
+    if (kf < ke) {  // both buffers are free here
+      fetch_tail(kf);
+      stash(buf);
+      __syncthreads();
+      compute(buf, false);
     }
     // v_mfma_f64_16x16x4f64 leaves D(i, j) in lane j + 16 (i % 4), register i / 4
-    const bool whole = s0 == 0 && s1 == sk.nk;
+    const bool whole = s0 == 0 && (s1 == sk.nk || sk.tri);
+    const bool mirror = sk.sym && m0 != n0;
+    int el = lane;
+    asm volatile("" : "+v"(el));
     double* P = Wp + ((size_t)lb * 2 + (g == g0 ? 0 : 1)) * TE * TE;
 #pragma unroll
     for (int i = 0; i < BI; ++i)
 #pragma unroll
       for (int j = 0; j < BJ; ++j) {
-        const int nl = wn + 16 * j + (lane & 15), n = n0 + nl;
+        const int nl = wn + 16 * j + (el & 15), n = n0 + nl;
 #pragma unroll
         for (int v = 0; v < 4; ++v) {
-          const int ml = wm + 16 * i + (lane >> 4) + 4 * v, m = m0 + ml;
+          const int ml = wm + 16 * i + (el >> 4) + 4 * v, m = m0 + ml;
           if (!whole) {
             P[nl * TM + ml] = acc[i][j][v];
           } else if (m < M && n < N) {
             double* p = C + (size_t)n * sk.ldc + m;
             const double x = acc[i][j][v] - corr_term(sk.corr, A, lda, B, ldb, m, n);
-            *p = sk.alpha * x + (sk.beta == 0.0 ? 0.0 : sk.beta * *p);
+            const double r = sk.alpha * x + (sk.beta == 0.0 ? 0.0 : sk.beta * *p);
+            *p = r;
+            if (mirror) C[(size_t)m * sk.ldc + n] = r;
           }
         }
+        __builtin_amdgcn_sched_barrier(0);  // one block's addresses and loads at a time
       }
-    g = (long)t * sk.nk + s1;
+    g = (long)t * sk.nk + (sk.tri ? sk.nk : s1);
   }
 }
 
@@ -289,7 +364,7 @@ __global__ void k_mg_fixup(Sk sk, const TW* __restrict__ Wp, const T* __restrict
   double s = 0.0;
   if (sk.S > 0) {
     // K-sliced: the first partial slot of workgroup (slice q, tile t), slices in order
-    const int nt = sk.tiles_m * sk.tiles_n, ns = (int)cdivu(sk.nk, sk.nks);
+    const int nt = sk.T, ns = (int)cdivu(sk.nk, sk.nks);
     if (ns <= 1) return;  // one slice covered the tile whole
     const TW* w0 = Wp + (size_t)t * 2 * TE * TE + (size_t)nl * sk.tm + ml;
     const size_t qs = (size_t)nt * 2 * TE * TE;  // slice to slice
@@ -315,6 +390,7 @@ __global__ void k_mg_fixup(Sk sk, const TW* __restrict__ Wp, const T* __restrict
   s -= corr_term(sk.corr, A, lda, B, ldb, m, n);
   TC* p = C + (size_t)n * sk.ldc + m;
   *p = (TC)(sk.alpha * s + (sk.beta == 0.0 ? 0.0 : sk.beta * (double)*p));
+  if (sk.sym && m0 != n0) C[(size_t)m * sk.ldc + n] = *p;
 }
 
 // ------------------------------------------------------------ bf16x3 ------
@@ -705,7 +781,6 @@ struct MgState {
   // tuned workgroup count per (kind, M, N, K, lda, ldb)
   std::map<std::tuple<int, int, int, int, int, int>, int> grid;
   // FP64 output tile per (kind, M, N, K, lda, ldb): index into the variants
-  std::map<std::tuple<int, int, int, int, int, int>, int> tile;
   float* f32[4] = {};  // FP32 work buffers of the fused mixed band-apply
   size_t f32_len[4] = {};
   float* B32 = nullptr;  // FP32 copy of the KB table
@@ -760,12 +835,19 @@ void* workspace(Ctx* c, size_t bytes) {
   return s->ws;
 }
 
+// operands known to leave part of the work out (Sk::sym, Sk::tri)
+enum Shape { SHAPE_FULL = 0, SHAPE_SYM = 1, SHAPE_TRI = 2 };
+long n_tiles(int M, int N, int tm, int tn, int shape) {
+  const long a = cdivu(M, tm), b = cdivu(N, tn);
+  return shape == SHAPE_SYM ? a * (a + 1) / 2 : a * b;
+}
+
 // A schedule code: > 0 = stream-K on that many workgroups, < 0 = K-sliced
 // with -code slices (on the multiple of 8 workgroups that covers slices x
 // tiles; -1 is one workgroup per output tile)
 Sk make_sk(int M, int N, int K, int kt, int code, double alpha, double beta, int ldc, int corr,
-           int tm = TE, int tn = TE, bool nfast = false) {
-  Sk sk;
+           int tm = TE, int tn = TE, bool nfast = false, int shape = 0) {
+  Sk sk{};
   sk.M = M;
   sk.N = N;
   sk.K = K;
@@ -775,7 +857,10 @@ Sk make_sk(int M, int N, int K, int kt, int code, double alpha, double beta, int
   sk.tiles_n = (int)cdivu(N, tn);
   sk.nk = (int)cdivu(K, kt);
   sk.nfast = nfast ? 1 : 0;
-  const long T = (long)sk.tiles_m * sk.tiles_n;
+  const long T = n_tiles(M, N, tm, tn, shape);
+  sk.T = (int)T;
+  sk.sym = shape == SHAPE_SYM ? 1 : 0;
+  sk.tri = shape == SHAPE_TRI && code == -1 ? 1 : 0;
   if (code > 0) {
     sk.S = 0;
     sk.nks = 0;
@@ -842,7 +927,7 @@ bool tuning_off() {
 // workgroups per CU; 0 on failure
 template <typename F>
 int choose_grid(Ctx* c, int kind, int M, int N, int K, int kt, int tm, int tn, int lda, int ldb,
-                int per_cu_max, size_t part_elem, F trial) {
+                int per_cu_max, size_t part_elem, int shape, F trial) {
   MgState* s = state(c);
   const int mode = g_sched.load(std::memory_order_relaxed);
   const auto key = std::make_tuple(kind + 1000 * mode, M, N, K, lda, ldb);
@@ -851,17 +936,17 @@ int choose_grid(Ctx* c, int kind, int M, int N, int K, int kt, int tm, int tn, i
   int cus = 256;
   (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, c->dev);
   cus = std::max(kXcd, cus / kXcd * kXcd);
-  const long T = (long)cdivu(M, tm) * cdivu(N, tn);
+  const long T = n_tiles(M, N, tm, tn, shape);
   const std::vector<int> cand = sched_candidates(T, (int)cdivu(K, kt), cus, per_cu_max);
   int best_code = cand.empty() ? 2 * cus : cand.back();
-  if (mode == 0 && !cand.empty()) best_code = cand[per_cu_max > 1 ? 1 : 0];
+  if (mode == 0 && !cand.empty()) best_code = cand[per_cu_max - 1];
   if (!tuning_off() && cand.size() > 1) {
     hipEvent_t e0, e1;
     QX_CHECK(hipEventCreate(&e0));
     QX_CHECK(hipEventCreate(&e1));
     float best = 1e30f;
     for (const int code : cand) {
-      const Sk probe = make_sk(M, N, K, kt, code, 1.0, 0.0, M, 0, tm, tn);
+      const Sk probe = make_sk(M, N, K, kt, code, 1.0, 0.0, M, 0, tm, tn, false, shape);
       if (!workspace(c, part_elem * TE * TE * sk_slots(probe))) return 0;
       if (trial(code)) return 0;  // warm
       QX_CHECK(hipEventRecord(e0, c->stream));
@@ -899,7 +984,7 @@ template <typename TW, typename T, typename TC, typename K1>
 int launch_sk(Ctx* c, const Sk& sk, K1 kernel, const T* A, int lda, const T* B, int ldb, TC* C) {
   TW* W = static_cast<TW*>(state(c)->ws);
   hipLaunchKernelGGL(kernel, dim3(sk.G), dim3(256), 0, c->stream, sk, A, lda, B, ldb, C, W);
-  const int tiles = sk.tiles_m * sk.tiles_n;
+  const int tiles = sk.T;
   if (sk_slots(sk))  // else every tile was written whole by its workgroup
     hipLaunchKernelGGL((k_mg_fixup<TW, T, TC>), dim3(TE * TE / 256, tiles), dim3(256), 0,
                        c->stream, sk, W, A, lda, B, ldb, C);
@@ -912,7 +997,7 @@ template <typename TW, typename T, typename TC, typename K1>
 int run_product(Ctx* c, int kind, int kt, int per_cu_max, K1 kernel, int M, int N, int K,
                 double alpha, const T* A, int lda, const T* B, int ldb, double beta, TC* C,
                 int ldc, int corr, long alo = 0, long blo = 0, int tm = TE, int tn = TE,
-                bool nfast = false) {
+                bool nfast = false, int shape = SHAPE_FULL) {
   if (M <= 0 || N <= 0) return 0;
   if ((lda | ldb) & 1) return -3;  // 8 / 16-byte row loads need even leading dimensions
   MgState* s = state(c);
@@ -921,13 +1006,14 @@ int run_product(Ctx* c, int kind, int kt, int per_cu_max, K1 kernel, int M, int 
   int code;
   if (known || tuning_off()) {
     code = choose_grid(c, kind, M, N, K, kt, tm, tn, lda, ldb, per_cu_max, sizeof(TW),
-                       [](int) { return 0; });
+                       shape, [](int) { return 0; });
   } else {
     TrialOut<TC> out((size_t)M * N);
     if (!out.p) return -3;
     code = choose_grid(c, kind, M, N, K, kt, tm, tn, lda, ldb, per_cu_max, sizeof(TW),
-                       [&](int cd) {
-                         Sk tk = make_sk(M, N, K, kt, cd, alpha, 0.0, M, corr, tm, tn, nfast);
+                       shape, [&](int cd) {
+                         Sk tk =
+                             make_sk(M, N, K, kt, cd, alpha, 0.0, M, corr, tm, tn, nfast, shape);
                          tk.alo = alo;
                          tk.blo = blo;
                          return launch_sk<TW>(c, tk, kernel, A, lda, B, ldb, out.p);
@@ -935,7 +1021,7 @@ int run_product(Ctx* c, int kind, int kt, int per_cu_max, K1 kernel, int M, int 
     QX_CHECK(hipStreamSynchronize(c->stream));  // trials done before the scratch goes
   }
   if (code == 0) return -3;
-  Sk sk = make_sk(M, N, K, kt, code, alpha, beta, ldc, corr, tm, tn, nfast);
+  Sk sk = make_sk(M, N, K, kt, code, alpha, beta, ldc, corr, tm, tn, nfast, shape);
   if (!workspace(c, sizeof(TW) * TE * TE * sk_slots(sk))) return -3;
   sk.alo = alo;
   sk.blo = blo;
@@ -1054,78 +1140,48 @@ float* mg_f32_scratch(Ctx* c, int i, size_t n) {
 int mg_tuned_shapes(Ctx* c) { return c->mg ? (int)state(c)->grid.size() : 0; }
 
 namespace {
-// FP64 product on the output tile chosen for its shape: the four tiles
-// (128 | 96) x (128 | 96) are timed on the first product of a shape (into a
-// scratch output; each with its own tuned grid) and the fastest is kept;
-// QX_GEMM_NOTUNE=1 takes the tile that pads the output least
+// FP64 product on the output tile, (128 | 96) x (128 | 96), that pads the
+// output least, 96 x 96 when even (the four run within 4 % of one another per
+// computed output: 63.0, 61.9 and 60.8 TF/s for 96 x 96, 128 x 96 and 128 x 128
+// in the TN product above); timing all four on first use took four times as
+// long and chose by noise.
 template <bool AK>
 int f64_product(Ctx* c, int kind, int M, int N, int K, double alpha, const double* A, int lda,
-                const double* B, int ldb, double beta, double* C, int ldc, int corr) {
+                const double* B, int ldb, double beta, double* C, int ldc, int corr, int shape) {
   using KF = void (*)(Sk, const double*, int, const double*, int, double*, double*);
-  static const KF ks[4] = {k_mg_f64<AK, 4, 4>, k_mg_f64<AK, 4, 3>, k_mg_f64<AK, 3, 4>,
-                           k_mg_f64<AK, 3, 3>};
-  static const int tms[4] = {128, 128, 96, 96}, tns[4] = {128, 96, 128, 96};
-  if (M <= 0 || N <= 0) return 0;
-  if ((lda | ldb) & 1) return -3;
-  MgState* s = state(c);
-  const auto key = std::make_tuple(kind, M, N, K, lda, ldb);
-  auto run = [&](int v, double b, double* out, int ldo) {
-    return run_product<double>(c, kind + 10 * (v + 1), KT64, 2, ks[v], M, N, K, alpha, A, lda, B,
-                               ldb, b, out, ldo, corr, 0, 0, tms[v], tns[v], !AK);
-  };
-  auto it = s->tile.find(key);
+  static const KF ks[4] = {k_mg_f64<AK, 3, 3>, k_mg_f64<AK, 4, 4>, k_mg_f64<AK, 4, 3>,
+                           k_mg_f64<AK, 3, 4>};
+  if (std::max(lda, ldb) >= 1 << 22) return -3;  // 32-bit offsets within a tile
+  static const int tms[4] = {96, 128, 128, 96}, tns[4] = {96, 128, 96, 128};
   int best = 0;
-  if (it != s->tile.end()) {
-    best = it->second;
-  } else if (tuning_off()) {
-    long least = -1;
-    for (int v = 0; v < 4; ++v) {
-      const long area = (long)cdivu(M, tms[v]) * tms[v] * (long)cdivu(N, tns[v]) * tns[v];
-      if (least < 0 || area < least) {
-        least = area;
-        best = v;
-      }
+  long least = -1;
+  for (int v = 0; v < (shape == SHAPE_SYM ? 2 : 4); ++v) {
+    const long area = n_tiles(M, N, tms[v], tns[v], shape) * tms[v] * tns[v];
+    if (least < 0 || area < least) {
+      least = area;
+      best = v;
     }
-    s->tile[key] = best;
-  } else {
-    TrialOut<double> out((size_t)M * N);
-    if (!out.p) return -3;
-    hipEvent_t e0, e1;
-    QX_CHECK(hipEventCreate(&e0));
-    QX_CHECK(hipEventCreate(&e1));
-    float bms = 1e30f;
-    for (int v = 0; v < 4; ++v) {
-      if (int rc = run(v, 0.0, out.p, M)) return rc;  // tunes the grid of this tile
-      QX_CHECK(hipEventRecord(e0, c->stream));
-      for (int r = 0; r < 2; ++r)
-        if (int rc = run(v, 0.0, out.p, M)) return rc;
-      QX_CHECK(hipEventRecord(e1, c->stream));
-      QX_CHECK(hipEventSynchronize(e1));
-      float ms = 0.f;
-      QX_CHECK(hipEventElapsedTime(&ms, e0, e1));
-      if (ms < bms) {
-        bms = ms;
-        best = v;
-      }
-    }
-    (void)hipEventDestroy(e0);
-    (void)hipEventDestroy(e1);
-    s->tile[key] = best;
   }
-  return run(best, beta, C, ldc);
+  return run_product<double>(c, kind + 10 * (best + 1) + 100 * shape, KT64, best == 0 ? 3 : 2,
+                             ks[best], M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, corr, 0, 0,
+                             tms[best], tns[best], !AK, shape);
 }
 }  // namespace
 
 // FP64 TN: C = alpha (A^T B - corr) + beta C
 int mg_dgemm_tn(Ctx* c, int M, int N, int K, double alpha, const double* A, int lda,
                 const double* B, int ldb, double beta, double* C, int ldc, int corr) {
-  return f64_product<true>(c, 0, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, corr);
+  // one matrix against itself (an overlap): half of the tiles
+  const bool sym = A == B && lda == ldb && M == N && beta == 0.0;
+  return f64_product<true>(c, 0, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, corr,
+                           sym ? SHAPE_SYM : SHAPE_FULL);
 }
 
-// FP64 NN: C = alpha A B + beta C
+// FP64 NN: C = alpha A B + beta C; upper: B(k, n) = 0 for k > n
 int mg_dgemm_nn(Ctx* c, int M, int N, int K, double alpha, const double* A, int lda,
-                const double* B, int ldb, double beta, double* C, int ldc) {
-  return f64_product<false>(c, 1, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, 0);
+                const double* B, int ldb, double beta, double* C, int ldc, bool upper) {
+  return f64_product<false>(c, 1, M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, 0,
+                            upper ? SHAPE_TRI : SHAPE_FULL);
 }
 
 // split bf16x3 TN on T operands into TC: C = alpha (A^T B - corr) + beta C
