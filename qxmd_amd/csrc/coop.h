@@ -86,9 +86,10 @@ __device__ inline double wave_sum(double v) {
 // 256 threads = 4 wavefronts, each a 32 x 32 quadrant as 2 x 2 blocks of
 // v_mfma_f64_16x16x4f64.  fa(m, k) and fb(k, n) return the operands, 0 out of
 // range, and must read a valid address for every m, n < 64 and k < K (they
-// load unconditionally from a clamped index and select, so that the loads of
-// a stage are all in flight together); K is walked 16 at a time through the
-// LDS tiles As/Bs.
+// load unconditionally from a clamped index and select).  K <= 64, and the loads
+// of all of it are issued first: agent-scope loads come from beyond the L1, and
+// waiting for them once per 16 k was most of a tile's time.  K is walked 16 at a
+// time through the LDS tiles As/Bs.
 typedef double dv4 __attribute__((ext_vector_type(4)));
 constexpr int kTileLd = 66;
 
@@ -105,25 +106,25 @@ struct Tile64 {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = (wave & 1) * 32, wn = (wave >> 1) * 32;
     const int m = tid >> 2, kk = (tid & 3) * 4;
-    double ra[4], rb[4];
-    auto fetch = [&](int k0) {
+    double ra[4][4], rb[4][4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
-        const int k = k0 + kk + u, kc = min(k, K - 1);
+        const int k = 16 * q + kk + u, kc = min(k, K - 1);
         const double va = fa(m, kc), vb = fb(kc, m);
-        ra[u] = k < K ? va : 0.0;
-        rb[u] = k < K ? vb : 0.0;
+        ra[q][u] = k < K ? va : 0.0;
+        rb[q][u] = k < K ? vb : 0.0;
       }
-    };
-    fetch(0);
-    for (int k0 = 0; k0 < K; k0 += 16) {
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      if (16 * q >= K) break;
 #pragma unroll
       for (int u = 0; u < 4; ++u) {
-        As[kk + u][m] = ra[u];
-        Bs[kk + u][m] = rb[u];
+        As[kk + u][m] = ra[q][u];
+        Bs[kk + u][m] = rb[q][u];
       }
       __syncthreads();
-      if (k0 + 16 < K) fetch(k0 + 16);  // next chunk in flight during the MFMAs
 #pragma unroll
       for (int k4 = 0; k4 < 16; k4 += 4) {
         const int kr = k4 + (lane >> 4), c = lane & 15;

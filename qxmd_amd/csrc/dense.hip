@@ -17,6 +17,7 @@
 #include <cstdlib>
 #include <vector>
 #include "context.h"
+#include "chol_wg.h"
 #include "coop.h"
 
 namespace qx {
@@ -229,53 +230,54 @@ __global__ void k_flag_to_ok(const int* fail, int* ok) { ok[0] = fail[0] ? 0 : 1
 //       inverse, X_bj = -X_bb T_bj (j < b);
 //   (C) the trailing update S_rc -= L_rb L_cb^T (b < c <= r) and the
 //       accumulation T_ij += L_ib X_bj (i > b, j <= b); the workgroup that
-//       owns the next diagonal tile factors and inverts it in LDS right after
+//       owns the next diagonal tile factors and inverts it right after
 //       its update (look-ahead), so block b+1 is ready at the barrier.
 // All matrix traffic goes through device-scope accesses (the tiles move
 // between workgroups on different XCDs).
 
-// diagonal block in LDS: P (lower part filled) -> L_bb, Q -> L_bb^-1 (column
-// sweep: row k of Q is final once divided by L_kk, then the rows below
-// subtract L_ik Q_k).  Written to s (lower) and x (full block, zeros above).
-__device__ void chol_diag_block(double* s, int n, int k0, int kb, double* x, int* fail,
-                                double (*P)[NBK + 1], double (*Q)[NBK + 1]) {
-  const int t = threadIdx.x;
-  for (int idx = t; idx < NBK * NBK; idx += blockDim.x) {
-    const int i = idx & (NBK - 1), j = idx / NBK;
-    if (!(i < kb && j < kb && i >= j)) P[i][j] = 0.0;
-    Q[i][j] = (i == j && i < kb) ? 1.0 : 0.0;
-  }
+// diagonal block: P (lower part filled, in LDS) -> X_bb = L_bb^-1 (the full block,
+// zeros above), factored in the registers of the workgroup: 64 steps of one
+// barrier each.  With the block in LDS and three barriers a step this was most
+// of the time of a block column; n = 540: 943 -> 427 us  fail[0] = 1 where a
+// pivot is not positive (dg = 0: no rounding bound, the pivots are those of a
+// Schur complement).
+__device__ inline void chol_diag_block(int n, int k0, int kb, double* x, int* fail,
+                                       double (*P)[NBK + 1]) {
+  using S = Shape<256, NBK / 16>;
+  __shared__ CholLds<S> L;
+  const int t = threadIdx.x, ti = t >> 4, tj = t & 15;
+  double A[S::NR][S::NC];
+#pragma unroll
+  for (int r = 0; r < S::NR; ++r)
+#pragma unroll
+    for (int c = 0; c < S::NC; ++c) {
+      const int i = ti + S::RW * r, j = tj + 16 * c;
+      A[r][c] = (i < kb && j < kb) ? P[max(i, j)][min(i, j)] : 0.0;
+      if (j == 0) {
+        L.src[0][i] = i == 0 ? 1.0 : A[r][c];
+        L.dg[i] = 0.0;
+      }
+    }
+  if (t == 0) L.piv[0] = A[0][0];
+  bool good = true;
+  chol_phase<S, 0>(A, L, kb, t, ti, tj, good);
   __syncthreads();
-  const int rr = t & 63, part = t >> 6;
-  for (int k = 0; k < kb; ++k) {
-    const double dkk = P[k][k];
-    const bool bad = !(dkk > 1e-30);
-    const double lkk = bad ? 0.0 : sqrt(dkk), il = bad ? 0.0 : 1.0 / lkk;
-    __syncthreads();
-    if (t == 0) {
-      P[k][k] = lkk;
-      if (bad) fail[0] = 1;
+#pragma unroll
+  for (int r = 0; r < S::NR; ++r) {
+    const int i = ti + S::RW * r;
+    const double il = i < kb ? sqrt(L.inv[i]) : 0.0;
+#pragma unroll
+    for (int c = 0; c < S::NC; ++c) {
+      const int j = tj + 16 * c;
+      if (i < kb && j < kb)
+        st_agent(&x[(size_t)(k0 + i) * n + (k0 + j)], j < i ? A[r][c] * il : j == i ? il : 0.0);
     }
-    if (t > k && t < kb) P[t][k] *= il;
-    if (t <= k) Q[k][t] *= il;
-    __syncthreads();
-    const int i = k + 1 + rr;
-    if (i < kb) {
-      const double lik = P[i][k];
-      for (int c = k + 1 + part; c <= i; c += 4) P[i][c] -= lik * P[c][k];
-      for (int c = part; c <= k; c += 4) Q[i][c] -= lik * Q[k][c];
-    }
-    __syncthreads();
   }
-  for (int idx = t; idx < kb * kb; idx += blockDim.x) {
-    const int i = idx % kb, j = idx / kb;
-    if (i >= j) st_agent(&s[(size_t)(k0 + i) + (size_t)n * (k0 + j)], P[i][j]);
-    st_agent(&x[(size_t)(k0 + i) * n + (k0 + j)], Q[i][j]);
-  }
+  if (t == 0 && !good) fail[0] = 1;
   __syncthreads();
 }
 
-constexpr size_t kCholLds = sizeof(double) * (32 * kTileLd + 2 * NBK * (NBK + 1));
+constexpr size_t kCholLds = sizeof(double) * (32 * kTileLd + NBK * (NBK + 1));
 
 __global__ void __launch_bounds__(256) k_chol_inv_coop(double* __restrict__ s, int n,
                                                        double* __restrict__ x, int* fail, int* bar,
@@ -284,7 +286,6 @@ __global__ void __launch_bounds__(256) k_chol_inv_coop(double* __restrict__ s, i
   auto As = reinterpret_cast<double (*)[kTileLd]>(smem);
   auto Bs = reinterpret_cast<double (*)[kTileLd]>(smem + 16 * kTileLd);
   auto P = reinterpret_cast<double (*)[NBK + 1]>(smem + 32 * kTileLd);
-  auto Q = reinterpret_cast<double (*)[NBK + 1]>(smem + 32 * kTileLd + NBK * (NBK + 1));
   const int G = gridDim.x, g = blockIdx.x, t = threadIdx.x;
   const int nblk = (n + NBK - 1) / NBK;
   int nbar = 0;
@@ -301,7 +302,7 @@ __global__ void __launch_bounds__(256) k_chol_inv_coop(double* __restrict__ s, i
     __syncthreads();
   }
   grid_barrier(bar, ++nbar * G, err);  // X zeroed before any block of it is written
-  if (g == 0) chol_diag_block(s, n, 0, min(NBK, n), x, fail, P, Q);
+  if (g == 0) chol_diag_block(n, 0, min(NBK, n), x, fail, P);
   grid_barrier(bar, ++nbar * G, err);
   for (int b = 0; b < nblk; ++b) {
     const int k0 = b * NBK, kb = min(NBK, n - k0);
@@ -367,7 +368,7 @@ __global__ void __launch_bounds__(256) k_chol_inv_coop(double* __restrict__ s, i
             if (m < nr && c < nc && m >= c) P[m][c] = ld_agent(S_(r0 + m, c0 + c)) - v;
           });
           __syncthreads();
-          chol_diag_block(s, n, r0, nr, x, fail, P, Q);
+          chol_diag_block(n, r0, nr, x, fail, P);
         } else {
           T.each([&](int m, int c, double v) {
             if (m < nr && c < nc) st_agent(S_(r0 + m, c0 + c), ld_agent(S_(r0 + m, c0 + c)) - v);
@@ -452,7 +453,8 @@ static int chol_inv_legacy(Ctx* c, double* s, int n, double* x, int* flag) {
   return 0;
 }
 
-// s: n x n column-major (lower valid; modified), x: n x n row-major output
+// s: n x n column-major (lower valid; overwritten, its diagonal blocks not by
+// L), x: n x n row-major output
 // L^-1; ok[0] = lcholesky, ok[1] = 1 if a grid barrier gave up.  flag:
 // device int scratch.
 int dense_chol_inv(Ctx* c, double* s, int n, double* x, int* ok, int* flag) {
