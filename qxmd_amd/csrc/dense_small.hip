@@ -217,18 +217,36 @@ __global__ void __launch_bounds__(S::T) k_tridiag_wg(double* __restrict__ a, int
       const int i = ti + S::RW * r, j = tj + 16 * c;
       A[r][c] = (i < n && j < n) ? a[(size_t)j + (size_t)n * i] : 0.0;
     }
+  // the largest element is brought to [1/2, 1) by a power of two: h is a square
+  // and u.(A u) a cube of the matrix's scale
+  __shared__ double wmax[S::T / 64];
+  double mx = 0.0;
+#pragma unroll
+  for (int r = 0; r < S::NR; ++r)
+#pragma unroll
+    for (int c = 0; c < S::NC; ++c) mx = fmax(mx, fabs(A[r][c]));
+  for (int o = 32; o > 0; o >>= 1) mx = fmax(mx, __shfl_xor(mx, o, 64));
+  if ((t & 63) == 0) wmax[t >> 6] = mx;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < S::T / 64; ++w) mx = fmax(mx, wmax[w]);
+  const int sh = -__builtin_amdgcn_frexp_exp(mx);
+#pragma unroll
+  for (int r = 0; r < S::NR; ++r)
+#pragma unroll
+    for (int c = 0; c < S::NC; ++c) A[r][c] = ldexp(A[r][c], sh);
   for (int i = t; i < S::NL; i += S::T) {
     const bool in = i > 0 && i < n;
-    L.xc[0][i] = make_double2(in ? a[i] : 0.0, in ? a[(size_t)n + i] : 0.0);
+    L.xc[0][i] =
+        make_double2(in ? ldexp(a[i], sh) : 0.0, in ? ldexp(a[(size_t)n + i], sh) : 0.0);
     L.xc[1][i] = make_double2(0.0, 0.0);
     L.q[i] = 0.0;
   }
   __syncthreads();
   trd_phase<S, 0>(A, L, n, t, ti, tj);
   // column n - 2 is the one published last
-  if (t < n) e[t] = t < n - 2 ? L.e[t] : t == n - 2 ? L.xc[n & 1][n - 1].x : 0.0;
-  for (int i = t + S::T; i < n; i += S::T)
-    e[i] = i < n - 2 ? L.e[i] : i == n - 2 ? L.xc[n & 1][n - 1].x : 0.0;
+  for (int i = t; i < n; i += S::T)
+    e[i] = ldexp(i < n - 2 ? L.e[i] : i == n - 2 ? L.xc[n & 1][n - 1].x : 0.0, -sh);
 #pragma unroll
   for (int c = 0; c < S::NC; ++c) {
     const int j = tj + 16 * c;
@@ -237,7 +255,7 @@ __global__ void __launch_bounds__(S::T) k_tridiag_wg(double* __restrict__ a, int
 #pragma unroll
     for (int r = 0; r < S::NR; ++r) {
       const int i = ti + S::RW * r;
-      if (i == j && i < n) d[i] = A[r][c];
+      if (i == j && i < n) d[i] = ldexp(A[r][c], -sh);
       if (i > j && i < n && j < n - 2) a[(size_t)i + (size_t)n * j] = A[r][c] * inv;
     }
   }
