@@ -118,6 +118,49 @@ static int get_reference(Ctx* c, const double* src, double* host, int nb) {
   return 0;
 }
 
+struct ReadSegs {
+  const unsigned* src[4];
+  unsigned words[4], at[4];
+};
+static __global__ void k_read_host(ReadSegs s, unsigned* __restrict__ out) {
+  const unsigned q = blockIdx.y;
+  for (unsigned i = blockIdx.x * blockDim.x + threadIdx.x; i < s.words[q];
+       i += gridDim.x * blockDim.x)
+    out[s.at[q] + i] = s.src[q][i];
+}
+
+int read_host(Ctx* c, std::initializer_list<HostRead> segs) {
+  ReadSegs s{};
+  unsigned n = 0, at = 0;
+  size_t total = 0;
+  for (const HostRead& r : segs) total += r.bytes;
+  const bool pinned = segs.size() <= 4 && total <= Ctx::kHostRead;
+  for (const HostRead& r : segs) {
+    if (!pinned) {
+      QX_CHECK(hipMemcpyAsync(r.dst, r.src, r.bytes, hipMemcpyDeviceToHost, c->stream));
+      continue;
+    }
+    s.src[n] = static_cast<const unsigned*>(r.src);
+    s.words[n] = (unsigned)(r.bytes / 4);
+    s.at[n++] = at;
+    at += (unsigned)(r.bytes / 4);
+  }
+  if (pinned && at) {
+    hipLaunchKernelGGL(k_read_host, dim3(4, n), dim3(256), 0, c->stream, s,
+                       reinterpret_cast<unsigned*>(c->d_hflag + 4));
+    QX_CHECK(hipGetLastError());
+  }
+  QX_CHECK(hipStreamSynchronize(c->stream));
+  if (pinned) {
+    const char* h = reinterpret_cast<const char*>(c->h_flag + 4);
+    for (const HostRead& r : segs) {
+      std::memcpy(r.dst, h, r.bytes);
+      h += r.bytes;
+    }
+  }
+  return 0;
+}
+
 int hpsi_batched(Ctx* c, const double* x, double* hx, int nb, int prec) {
   if (prec == PREC_FP32) {
     const int rf = hpsi_mixed_fused(c, x, hx, nb);
@@ -152,8 +195,7 @@ int schmidt_dev(Ctx* c, double* psi, int nb, int* ok_host, int prec, bool split_
   if (rc) return rc;
   if ((rc = dense_chol_inv(c, S, nb, Linv, ok, flag))) return rc;
   int okh[2] = {0, 0};
-  QX_CHECK(hipMemcpyAsync(okh, ok, 2 * sizeof(int), hipMemcpyDeviceToHost, c->stream));
-  QX_CHECK(hipStreamSynchronize(c->stream));
+  if ((rc = read_host(c, {{okh, ok, 2 * sizeof(int)}}))) return rc;
   if (okh[1]) return -20;  // a grid barrier of the Cholesky gave up
   *ok_host = okh[0];
   if (!okh[0]) return 0;
@@ -206,11 +248,7 @@ static int rotate_dev(Ctx* c, double* psi, double* hpsi, int nb, double* eig_hos
     QX_CHECK(hipMemcpyAsync(hpsi, out, sizeof(double) * (size_t)n * nb, hipMemcpyDeviceToDevice,
                             c->stream));
   }
-  if (eig_host) {
-    QX_CHECK(hipMemcpyAsync(eig_host, w, sizeof(double) * nb, hipMemcpyDeviceToHost, c->stream));
-    QX_CHECK(hipStreamSynchronize(c->stream));
-  }
-  return 0;
+  return eig_host ? read_host(c, {{eig_host, w, sizeof(double) * nb}}) : 0;
 }
 
 // ekib: 2 <psi|T|psi> per band (ekinetic2, Sources/engrad.f90:117-122)
@@ -319,7 +357,8 @@ int qx_create(qx_ctx** out, int n1, int n2, int n3, int nplw, const int* nga, co
   c->bb_nch = c->nplwex / kBbChunk + 1;
   QX_CHECK(hipMalloc(&c->d_bb, sizeof(double) * (32 + 5 * (size_t)(c->bb_nch + 1))));
   QX_CHECK(hipMemset(c->d_bb, 0, sizeof(double) * (32 + 5 * (size_t)(c->bb_nch + 1))));
-  QX_CHECK(hipHostMalloc(reinterpret_cast<void**>(&c->h_flag), sizeof(int) * 4, hipHostMallocDefault));
+  QX_CHECK(hipHostMalloc(reinterpret_cast<void**>(&c->h_flag), sizeof(int) * 4 + Ctx::kHostRead,
+                         hipHostMallocDefault));
   QX_CHECK(hipHostGetDevicePointer(reinterpret_cast<void**>(&c->d_hflag), c->h_flag, 0));
   for (auto& e : c->ev) QX_CHECK(hipEventCreate(&e));
   for (auto& e : c->pev) QX_CHECK(hipEventCreate(&e));
@@ -630,8 +669,7 @@ int qx_ekib_slot(qx_ctx* h, int slot, int nb, double* ekib_host) {
                      c->d_slot[slot], t, c->d_kin, n, nb);
   pdot_batched(c, t, c->d_slot[slot], nb, d);
   std::vector<double> e(nb);
-  QX_CHECK(hipMemcpyAsync(e.data(), d, sizeof(double) * nb, hipMemcpyDeviceToHost, c->stream));
-  QX_CHECK(hipStreamSynchronize(c->stream));
+  if (int rc = read_host(c, {{e.data(), d, sizeof(double) * nb}})) return rc;
   for (int b = 0; b < nb; ++b) ekib_host[b] = 2.0 * e[b];
   return 0;
 }

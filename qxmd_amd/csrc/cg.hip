@@ -723,12 +723,12 @@ int bkl_band_by_band(Ctx* c, double* psi, double* hpsi, int nb, const double* ek
       if (!*static_cast<volatile int*>(c->h_flag)) break;
     }
   }
-  QX_CHECK(hipMemcpyAsync(eig, eig_d, sizeof(double) * nb, hipMemcpyDeviceToHost, c->stream));
   std::vector<double> bz(nb);
   std::vector<int> itv(nb);
-  QX_CHECK(hipMemcpyAsync(bz.data(), bz_d, sizeof(double) * nb, hipMemcpyDeviceToHost, c->stream));
-  QX_CHECK(hipMemcpyAsync(itv.data(), it_d, sizeof(int) * nb, hipMemcpyDeviceToHost, c->stream));
-  QX_CHECK(hipStreamSynchronize(c->stream));
+  if (int rc = read_host(c, {{eig, eig_d, sizeof(double) * nb},
+                             {bz.data(), bz_d, sizeof(double) * nb},
+                             {itv.data(), it_d, sizeof(int) * nb}}))
+    return rc;
   for (int b = 0; b < nb; ++b) {
     if (bzan) bzan[b] = bz[b];
     if (nriter) nriter[b] = itv[b];
@@ -995,12 +995,13 @@ int bkl_batched(Ctx* c, double* psi, double* hpsi, int nb, const double* ekib_ho
       return rc;
     }
   }
-  QX_CHECK(hipMemcpyAsync(eig_host, s.eig, sizeof(double) * nb, hipMemcpyDeviceToHost, c->stream));
-  if (bzan)
-    QX_CHECK(hipMemcpyAsync(bzan, s.zansa, sizeof(double) * nb, hipMemcpyDeviceToHost, c->stream));
   std::vector<int> itv(nb);
-  QX_CHECK(hipMemcpyAsync(itv.data(), s.iter, sizeof(int) * nb, hipMemcpyDeviceToHost, c->stream));
-  QX_CHECK(hipStreamSynchronize(c->stream));
+  std::vector<double> bz(nb);
+  if ((rc = read_host(c, {{eig_host, s.eig, sizeof(double) * nb},
+                          {bz.data(), s.zansa, sizeof(double) * nb},
+                          {itv.data(), s.iter, sizeof(int) * nb}})))
+    return rc;
+  if (bzan) std::copy(bz.begin(), bz.end(), bzan);
   if (nriter)
     for (int b = 0; b < nb; ++b) nriter[b] = itv[b];
   return 0;

@@ -1,5 +1,6 @@
 // context.h -- device-resident plane-wave context of the qxmd_amd library.
 #pragma once
+#include <initializer_list>
 #include <hip/hip_runtime.h>
 #include <vector>
 #include "common.h"
@@ -85,13 +86,15 @@ struct Ctx {
   double *d_scal = nullptr;               // scalar work (device)
   int* d_sync = nullptr;                  // grid-barrier counter and error flags
   double* d_dwork = nullptr;              // dense eigensolver work (8 nbmax^2 + ...)
-  double* d_frc = nullptr;                // workspace of the nonlocal forces
+  double* d_frc = nullptr;                // workspace of the force calls
   size_t frc_len = 0;
   double* d_gs = nullptr;                 // K-slice partials of the small products
   size_t gs_len = 0;
   double* d_bb = nullptr;                 // band-by-band CG: scalars, then chunk sums
   int bb_nch = 0;                         // chunks of kBbChunk the chunk-sum space holds
-  int *h_flag = nullptr, *d_hflag = nullptr;  // pinned host flag and its device address
+  // pinned host memory and its device address: 4 flag words, then kHostRead bytes
+  int *h_flag = nullptr, *d_hflag = nullptr;
+  static constexpr size_t kHostRead = 65536;
   size_t dwork_len = 0;
   hipEvent_t ev[8] = {};
   hipEvent_t pev[6] = {};                 // SCF band-step phase timers
@@ -389,6 +392,18 @@ int gemm_tn(Ctx* c, int M, int N, int K, double alpha, const double* A, int lda,
             int ldb, double beta, double* C, int ldc, int corr);
 int gemm_nn(Ctx* c, int M, int N, int K, double alpha, const double* A, int lda, const double* B,
             int ldb, double beta, double* C, int ldc, bool upper = false);
+// Results the host waits for (energies, eigenvalues, flags): the segments are
+// written to pinned memory by one kernel and copied out after a synchronisation
+// of the stream, 15 us where each hipMemcpyAsync to pageable memory and its
+// synchronisation took 45.  Sizes are multiples of 4 bytes; what exceeds the
+// pinned buffer or four segments goes through hipMemcpyAsync.
+struct HostRead {
+  void* dst;
+  const void* src;
+  size_t bytes;
+};
+int read_host(Ctx* c, std::initializer_list<HostRead> segs);
+double* call_workspace(Ctx* c, size_t n);
 // the products with a dimension of the output below 256 (gemm_small.hip), in
 // either precision, over `batch` operands at the given strides; rscale: a
 // factor per row m of C (TN)

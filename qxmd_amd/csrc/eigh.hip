@@ -963,8 +963,7 @@ int dense_eigh(Ctx* c, double* a, int n, double* z, double* w, double* work, int
   // together by CholeskyQR (scratch X).
   hipLaunchKernelGGL(k_cluster_scan, dim3(1), dim3(1024), 0, st, w, n, bounds, cl);
   int maxcl = 0;
-  QX_CHECK(hipMemcpyAsync(&maxcl, cl + n, sizeof(int), hipMemcpyDeviceToHost, st));
-  QX_CHECK(hipStreamSynchronize(st));
+  if (int rc = read_host(c, {{&maxcl, cl + n, sizeof(int)}})) return rc;
   const bool local = maxcl <= kClusterMax && std::getenv("QX_EIGH_CHOLQR") == nullptr;
   const dim3 tgrid((n + 31) / 32, (n + 31) / 32);
   for (int pass = 0; pass < 2; ++pass) {
@@ -990,8 +989,7 @@ int dense_eigh(Ctx* c, double* a, int n, double* z, double* w, double* work, int
   hipLaunchKernelGGL(k_sync_take, dim3(1), dim3(1), 0, st, c->d_sync, sflag);
   QX_CHECK(hipGetLastError());
   int hflags[17];
-  QX_CHECK(hipMemcpyAsync(hflags, ok, sizeof(int) * 17, hipMemcpyDeviceToHost, st));
-  QX_CHECK(hipStreamSynchronize(st));
+  if (int rc = read_host(c, {{hflags, ok, sizeof(int) * 17}})) return rc;
   if (hflags[16]) return -20;  // a grid barrier gave up
   // a Gram matrix of the re-orthonormalisation was not positive definite
   if (!local && (!hflags[0] || !hflags[2] || !hflags[4] || !hflags[8] || !hflags[10])) return -23;

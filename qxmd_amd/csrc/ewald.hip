@@ -156,13 +156,13 @@ int ewald_run(Ctx* c, const std::vector<EwIon>& ions, const Tab& tb, std::vector
   recolmb = 0.0;
   if (nion == 0 || numk2 == 0) return 0;
   const int nchunk = (int)cdivu(numk2, kEwChunk);
-  EwIon* d_ions = nullptr;
-  double *d_sf = nullptr, *d_et = nullptr, *d_part = nullptr, *d_out = nullptr;
-  QX_CHECK(hipMalloc(&d_ions, sizeof(EwIon) * nion));
-  QX_CHECK(hipMalloc(&d_sf, sizeof(double) * 2 * numk2));
-  QX_CHECK(hipMalloc(&d_et, sizeof(double) * numk2));
-  QX_CHECK(hipMalloc(&d_part, sizeof(double) * 4 * (size_t)nion * nchunk));
-  QX_CHECK(hipMalloc(&d_out, sizeof(double) * (4 * (size_t)nion + 1)));
+  const size_t n_part = 4 * (size_t)nion * nchunk, n_out = 4 * (size_t)nion + 1;
+  const size_t n_ions = (sizeof(EwIon) * nion + 15) / 16 * 2;  // doubles, 16-byte rounded
+  double* d_sf = call_workspace(c, 2 * (size_t)numk2 + n_ions + numk2 + n_part + n_out);
+  if (!d_sf) return -3;
+  EwIon* d_ions = reinterpret_cast<EwIon*>(d_sf + 2 * (size_t)numk2);
+  double* d_et = d_sf + 2 * (size_t)numk2 + n_ions;
+  double *d_part = d_et + numk2, *d_out = d_part + n_part;
   QX_CHECK(hipMemcpyAsync(d_ions, ions.data(), sizeof(EwIon) * nion, hipMemcpyHostToDevice,
                           c->stream));
   const double pi = std::acos(-1.0);
@@ -176,16 +176,9 @@ int ewald_run(Ctx* c, const std::vector<EwIon>& ions, const Tab& tb, std::vector
                      c->stream, d_part, nchunk, nion, d_et, numk2, d_out);
   QX_CHECK(hipGetLastError());
   std::vector<double> out(4 * (size_t)nion + 1);
-  QX_CHECK(hipMemcpyAsync(out.data(), d_out, sizeof(double) * out.size(), hipMemcpyDeviceToHost,
-                          c->stream));
-  QX_CHECK(hipStreamSynchronize(c->stream));
+  if (int rc = read_host(c, {{out.data(), d_out, sizeof(double) * out.size()}})) return rc;
   std::copy(out.begin(), out.begin() + 4 * nion, acc.begin());
   recolmb = out[4 * nion];
-  (void)hipFree(d_ions);
-  (void)hipFree(d_sf);
-  (void)hipFree(d_et);
-  (void)hipFree(d_part);
-  (void)hipFree(d_out);
   return 0;
 }
 

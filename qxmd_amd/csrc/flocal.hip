@@ -168,11 +168,11 @@ int flocal_sums(Ctx* c, const std::vector<Ion>& ions, const double* tab, int ld,
   sums.assign(3 * (size_t)nion, 0.0);
   if (nion == 0 || nplw5 < 1) return 0;
   const int nchunk = (int)cdivu(nplw5, kFlChunk);
-  Ion* d_ions = nullptr;
-  double *d_part = nullptr, *d_out = nullptr;
-  QX_CHECK(hipMalloc(&d_ions, sizeof(Ion) * nion));
-  QX_CHECK(hipMalloc(&d_part, sizeof(double) * 3 * (size_t)nion * nchunk));
-  QX_CHECK(hipMalloc(&d_out, sizeof(double) * 3 * (size_t)nion));
+  const size_t n_ions = (sizeof(Ion) * nion + 15) / 16 * 2;  // doubles, 16-byte rounded
+  double* ws = call_workspace(c, n_ions + 3 * (size_t)nion * (nchunk + 1));
+  if (!ws) return -3;
+  Ion* d_ions = reinterpret_cast<Ion*>(ws);
+  double *d_part = ws + n_ions, *d_out = d_part + 3 * (size_t)nion * nchunk;
   QX_CHECK(hipMemcpyAsync(d_ions, ions.data(), sizeof(Ion) * nion, hipMemcpyHostToDevice,
                           c->stream));
   hipLaunchKernelGGL(k_flocal, dim3(nchunk, cdivu(nion, kFlAtoms)), dim3(kFlThreads), 0,
@@ -182,13 +182,7 @@ int flocal_sums(Ctx* c, const std::vector<Ion>& ions, const double* tab, int ld,
   hipLaunchKernelGGL(k_flocal_sum, dim3(cdivu(3L * nion, 256)), dim3(256), 0, c->stream, d_part,
                      nchunk, nion, d_out);
   QX_CHECK(hipGetLastError());
-  QX_CHECK(hipMemcpyAsync(sums.data(), d_out, sizeof(double) * 3 * nion, hipMemcpyDeviceToHost,
-                          c->stream));
-  QX_CHECK(hipStreamSynchronize(c->stream));
-  (void)hipFree(d_ions);
-  (void)hipFree(d_part);
-  (void)hipFree(d_out);
-  return 0;
+  return read_host(c, {{sums.data(), d_out, sizeof(double) * 3 * nion}});
 }
 
 // floc(:, ia) = 2 (floc(:, ia) + sum) per type, as 1103-1116

@@ -105,8 +105,9 @@ __global__ void k_force_atoms(const double* __restrict__ T, const double* __rest
 
 }  // namespace
 
-// grown on demand and kept (a force evaluation per MD step); null when out of memory
-static double* frc_workspace(Ctx* c, size_t n) {
+// n doubles for the length of a force call: grown on demand and kept for the next
+// MD step's (a call ends synchronised); null when out of memory
+double* call_workspace(Ctx* c, size_t n) {
   if (c->frc_len < n) {
     if (c->d_frc) (void)hipFree(c->d_frc);  // waits for what still reads it
     c->d_frc = nullptr;
@@ -143,7 +144,7 @@ int kb_forces(Ctx* c, const double* psi, int nb, const double* occ_host, const d
   const size_t o_occ = 3 * (size_t)np, o_f = o_occ + nb, o_p0 = o_f + 3 * (size_t)c->natom;
   const size_t o_g = o_p0 + (p0.size() + 1) / 2, o_z = (o_g + 3 * (size_t)np + 1) / 2 * 2;
   const size_t o_t = o_z + (size_t)npj * nb, o_y = (o_t + 3 * (size_t)npj * kFrcParts + 1) / 2 * 2;
-  double* w = frc_workspace(c, o_y + own_y);
+  double* w = call_workspace(c, o_y + own_y);
   if (!w) return -3;
   QX_CHECK(hipMemcpyAsync(w, gx, sizeof(double) * np, hipMemcpyHostToDevice, c->stream));
   QX_CHECK(hipMemcpyAsync(w + np, gy, sizeof(double) * np, hipMemcpyHostToDevice, c->stream));
@@ -170,10 +171,7 @@ int kb_forces(Ctx* c, const double* psi, int nb, const double* occ_host, const d
   hipLaunchKernelGGL(k_force_atoms, dim3(cdivu(3L * c->natom, 256)), dim3(256), 0, c->stream, T,
                      c->d_D, reinterpret_cast<const int*>(w + o_p0), c->natom, npj, w + o_f);
   QX_CHECK(hipGetLastError());
-  QX_CHECK(hipMemcpyAsync(fnlc_host, w + o_f, sizeof(double) * 3 * c->natom,
-                          hipMemcpyDeviceToHost, c->stream));
-  QX_CHECK(hipStreamSynchronize(c->stream));
-  return 0;
+  return read_host(c, {{fnlc_host, w + o_f, sizeof(double) * 3 * c->natom}});
 }
 
 }  // namespace qx

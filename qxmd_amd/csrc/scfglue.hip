@@ -460,9 +460,7 @@ int mix_dev(Ctx* c, int lreset, double aslh, double bslh, int lmixhold) {
       hipLaunchKernelGGL(k_red_final, dim3(1), dim3(kRedThreads), 0, c->stream, S.d_red, nblk,
                          kPlMax, kntchg, 0, S.rvol, d_out);
       QX_CHECK(hipGetLastError());
-      QX_CHECK(hipMemcpyAsync(a.data(), d_out, sizeof(double) * kntchg, hipMemcpyDeviceToHost,
-                              c->stream));
-      QX_CHECK(hipStreamSynchronize(c->stream));
+      if (int rr = read_host(c, {{a.data(), d_out, sizeof(double) * kntchg}})) return rr;
       for (int i1 = 0; i1 < kntchg; ++i1) {
         A(i1, k) = a[i1];
         A(k, i1) = a[i1];
@@ -551,8 +549,7 @@ int potential_dev(Ctx* c, double* ene) {
   QX_CHECK(hipGetLastError());
   if ((rc = fast_permute_v(c))) return rc;
   double e[kNe];
-  QX_CHECK(hipMemcpyAsync(e, d_out, sizeof(e), hipMemcpyDeviceToHost, c->stream));
-  QX_CHECK(hipStreamSynchronize(c->stream));
+  if ((rc = read_host(c, {{e, d_out, sizeof(e)}}))) return rc;
   if (ene)
     for (int k = 0; k < kNe; ++k) ene[k] = e[k];
   return 0;
