@@ -367,10 +367,16 @@ __global__ void __launch_bounds__(256) k_bisect_ms(const double* __restrict__ d,
 // One thread per eigenvalue j: factor T - lambda_j I (partial pivoting, rows i
 // and i+1 swapped when the subdiagonal dominates), then solve with the column
 // j of X (row-major, X[i*n + j]) as right-hand side, in place, and normalise.
-// first != 0: the right-hand side is a fixed pseudo-random vector instead.
-// The running row of the factorisation and of the forward sweep stay in
-// registers, so every global access is independent of the recurrence.
-// lu: 5 n^2 doubles, entry (q, i) of thread j at lu[(q*n + i)*n + j].
+// first != 0: the right-hand side is a fixed pseudo-random vector instead, and
+// its forward sweep runs along with the factorisation.  lu: 5 n^2 doubles, entry
+// (q, i) of thread j at lu[(q*n + i)*n + j].
+//
+// There are too few threads to hide anything (160 are three wavefronts), so the
+// chains are kept short: one reciprocal per row serves the multiplier and, stored
+// in the place of the pivot, the back substitution; d and e come from LDS; the
+// sweeps load chunks of kIvChunk rows while the previous chunk is worked on (the
+// solution overwrites the right-hand side in place, so the compiler cannot hoist
+// the loads on its own).  n = 160, both passes: 181 -> 100 us.
 __device__ inline double inviter_start(int i, int j) {
   unsigned h = (unsigned)(i * 2654435761u) ^ (unsigned)(j * 40503u + 12345u);
   h ^= h >> 13;
@@ -379,28 +385,38 @@ __device__ inline double inviter_start(int i, int j) {
   return 0.5 + (double)(h & 0xffff) / 65536.0;
 }
 
-// Loads are gathered 32 steps at a time into registers ahead of the
-// recurrence (the solution overwrites the right-hand side in place, so the
-// compiler cannot hoist them on its own).
-constexpr int kIvChunk = 32;
+constexpr int kIvChunk = 16;
 
+template <bool STAGED>  // d and e in LDS (n <= kBisectLds)
 __global__ void __launch_bounds__(64) k_inviter_par(const double* __restrict__ d,
                                                     const double* __restrict__ e, int n,
                                                     const double* __restrict__ w,
                                                     const double* __restrict__ bounds,
                                                     double* __restrict__ lu,
                                                     double* __restrict__ X, int first) {
+  __shared__ double ds[STAGED ? kBisectLds : 1], es[STAGED ? kBisectLds : 1];
+  if (STAGED && first) {
+    for (int i = threadIdx.x; i < n; i += 64) {
+      ds[i] = d[i];
+      es[i] = i < n - 1 ? e[i] : 0.0;
+    }
+    __syncthreads();
+  }
   const int j = blockIdx.x * blockDim.x + threadIdx.x;
   if (j >= n) return;
   const size_t nn = (size_t)n * n;
-  double* dd = lu + j;           // U diagonal (tiny pivots replaced by +-pert)
-  double* du = dd + nn;          // U superdiagonal
+  double* rd = lu + j;           // reciprocals of the U diagonal (tiny ones +-pert)
+  double* du = rd + nn;          // U superdiagonal
   double* du2 = du + nn;         // U second superdiagonal
   double* dl = du2 + nn;         // multipliers
   double* pv = dl + nn;          // 1 when rows i, i+1 were swapped
+  double* x = X + j;
 #define L_(arr, i) arr[(size_t)(i) * n]
+  constexpr int CH = kIvChunk;
   if (first) {
-    // factor T - lambda I once; the second pass reuses it
+    // factor T - lambda I once (the second pass reuses it), L y = P b with it
+    auto dat = [&](int i) { return STAGED ? ds[i] : d[i]; };
+    auto eat = [&](int i) { return STAGED ? es[i] : e[i]; };
     const double eps = 2.220446049250313e-16;
     const double pert = eps * bounds[3];
     double lam = w[j];
@@ -408,83 +424,82 @@ __global__ void __launch_bounds__(64) k_inviter_par(const double* __restrict__ d
     for (int q = j; q > 0 && w[q] - w[q - 1] < 10.0 * eps * fabs(w[q]); --q) ++r;
     lam += (double)r * 10.0 * eps * fabs(lam);
     auto guard = [&](double v) { return fabs(v) < pert ? (v < 0.0 ? -pert : pert) : v; };
-    double dc = d[0] - lam, uc = n > 1 ? e[0] : 0.0;  // current row: diagonal, superdiagonal
+    double dc = dat(0) - lam, uc = n > 1 ? eat(0) : 0.0;  // current row: diagonal, superdiagonal
+    double xc = inviter_start(0, j);
     for (int i = 0; i < n - 1; ++i) {
-      const double sub = e[i];
-      const double dn = d[i + 1] - lam;
-      const double un = i + 2 < n ? e[i + 1] : 0.0;
-      if (fabs(dc) >= fabs(sub)) {
-        const double f = dc != 0.0 ? sub / dc : 0.0;
-        L_(dd, i) = guard(dc);
-        L_(du, i) = uc;
-        L_(du2, i) = 0.0;
-        L_(dl, i) = f;
-        L_(pv, i) = 0.0;
-        dc = dn - f * uc;
-        uc = un;
-      } else {
-        const double f = dc / sub;
-        L_(dd, i) = guard(sub);
-        L_(du, i) = dn;
-        L_(du2, i) = un;
-        L_(dl, i) = f;
-        L_(pv, i) = 1.0;
-        dc = uc - f * dn;
-        uc = -f * un;
-      }
+      const double sub = eat(i), dn = dat(i + 1) - lam, un = i + 2 < n ? eat(i + 1) : 0.0;
+      const double xr = inviter_start(i + 1, j);
+      const bool swap = !(fabs(dc) >= fabs(sub));
+      const double den = swap ? sub : dc, num = swap ? dc : sub;
+      const double rp = 1.0 / guard(den);
+      const double f = den != 0.0 ? num * rp : 0.0;
+      L_(rd, i) = rp;
+      L_(du, i) = swap ? dn : uc;
+      L_(du2, i) = swap ? un : 0.0;
+      L_(dl, i) = f;
+      L_(pv, i) = swap ? 1.0 : 0.0;
+      L_(x, i) = swap ? xr : xc;
+      xc = swap ? xc - f * xr : xr - f * xc;
+      dc = swap ? uc - f * dn : dn - f * uc;
+      uc = swap ? -f * un : un;
     }
-    L_(dd, n - 1) = guard(dc);
+    L_(rd, n - 1) = 1.0 / guard(dc);
     L_(du, n - 1) = 0.0;
     L_(du2, n - 1) = 0.0;
-  }
-  double* x = X + j;
-  // forward sweep L y = P b, the row being eliminated carried in xc
-  double xc = first ? inviter_start(0, j) : L_(x, 0);
-  for (int i0 = 0; i0 < n - 1; i0 += kIvChunk) {
-    double xr[kIvChunk], fr[kIvChunk], pr[kIvChunk];
+    L_(x, n - 1) = xc;
+  } else {
+    // forward sweep L y = P b, the row being eliminated carried in xc
+    double xc = L_(x, 0);
+    double xr[2][CH], fr[2][CH], pr[2][CH];
+    auto load = [&](int i0, double(&xq)[CH], double(&fq)[CH], double(&pq)[CH]) {
 #pragma unroll
-    for (int c = 0; c < kIvChunk; ++c) {
-      const int i = i0 + c;
-      if (i < n - 1) {
-        xr[c] = first ? inviter_start(i + 1, j) : L_(x, i + 1);
-        fr[c] = L_(dl, i);
-        pr[c] = L_(pv, i);
+      for (int c = 0; c < CH; ++c) {
+        const int i = min(i0 + c, n - 2);
+        xq[c] = L_(x, i + 1);
+        fq[c] = L_(dl, i);
+        pq[c] = L_(pv, i);
       }
-    }
+    };
+    auto sweep = [&](int i0, double(&xq)[CH], double(&fq)[CH], double(&pq)[CH]) {
 #pragma unroll
-    for (int c = 0; c < kIvChunk; ++c) {
-      const int i = i0 + c;
-      if (i < n - 1) {
-        if (pr[c] == 0.0) {
-          L_(x, i) = xc;
-          xc = xr[c] - fr[c] * xc;
-        } else {
-          L_(x, i) = xr[c];
-          xc = xc - fr[c] * xr[c];
+      for (int c = 0; c < CH; ++c)
+        if (i0 + c < n - 1) {
+          const bool swap = pq[c] != 0.0;
+          L_(x, i0 + c) = swap ? xq[c] : xc;
+          xc = swap ? xc - fq[c] * xq[c] : xq[c] - fq[c] * xc;
         }
+    };
+    if (n > 1) {
+      load(0, xr[0], fr[0], pr[0]);
+      for (int i0 = 0; i0 < n - 1; i0 += 2 * CH) {
+        load(i0 + CH, xr[1], fr[1], pr[1]);
+        sweep(i0, xr[0], fr[0], pr[0]);
+        load(i0 + 2 * CH, xr[0], fr[0], pr[0]);
+        sweep(i0 + CH, xr[1], fr[1], pr[1]);
       }
     }
+    L_(x, n - 1) = xc;
   }
-  L_(x, n - 1) = xc;
   // back substitution U x = y, with the squared norm accumulated on the way
   double x1 = 0.0, x2 = 0.0, big = 0.0, s2 = 0.0;  // x1 = x[i+1], x2 = x[i+2]
-  for (int i1 = n - 1; i1 >= 0; i1 -= kIvChunk) {
-    double yr[kIvChunk], ur[kIvChunk], u2r[kIvChunk], dr[kIvChunk];
+  double yr[2][CH], ur[2][CH], u2r[2][CH], rr[2][CH];
+  auto load = [&](int i1, double(&y)[CH], double(&u)[CH], double(&v)[CH], double(&r)[CH]) {
 #pragma unroll
-    for (int c = 0; c < kIvChunk; ++c) {
-      const int i = i1 - c;
-      if (i >= 0) {
-        yr[c] = L_(x, i);
-        ur[c] = L_(du, i);
-        u2r[c] = L_(du2, i);
-        dr[c] = L_(dd, i);
-      }
+    for (int c = 0; c < CH; ++c) {
+      const int i = max(i1 - c, 0);
+      y[c] = L_(x, i);
+      u[c] = L_(du, i);
+      v[c] = L_(du2, i);
+      r[c] = L_(rd, i);
     }
+  };
+  auto back = [&](int i1, double(&y)[CH], double(&u)[CH], double(&u2)[CH], double(&r)[CH],
+                  double(&ynext)[CH]) {
 #pragma unroll
-    for (int c = 0; c < kIvChunk; ++c) {
+    for (int c = 0; c < CH; ++c) {
       const int i = i1 - c;
       if (i >= 0) {
-        const double v = (yr[c] - ur[c] * x1 - u2r[c] * x2) / dr[c];
+        const double v = (y[c] - u[c] * x1 - u2[c] * x2) * r[c];
         L_(x, i) = v;
         x2 = x1;
         x1 = v;
@@ -492,11 +507,13 @@ __global__ void __launch_bounds__(64) k_inviter_par(const double* __restrict__ d
         big = fmax(big, fabs(v));
         if (big > 1e150) {
           // rescale the solved part, the right-hand side still in memory and
-          // the part of it already in registers
+          // the parts of it already in registers
           for (int q = 0; q < n; ++q) L_(x, q) *= 1e-150;
 #pragma unroll
-          for (int c2 = 0; c2 < kIvChunk; ++c2)
-            if (c2 > c) yr[c2] *= 1e-150;
+          for (int c2 = 0; c2 < CH; ++c2) {
+            if (c2 > c) y[c2] *= 1e-150;
+            ynext[c2] *= 1e-150;
+          }
           x1 *= 1e-150;
           x2 *= 1e-150;
           s2 *= 1e-300;
@@ -504,16 +521,23 @@ __global__ void __launch_bounds__(64) k_inviter_par(const double* __restrict__ d
         }
       }
     }
+  };
+  load(n - 1, yr[0], ur[0], u2r[0], rr[0]);
+  for (int i1 = n - 1; i1 >= 0; i1 -= 2 * CH) {
+    load(i1 - CH, yr[1], ur[1], u2r[1], rr[1]);
+    back(i1, yr[0], ur[0], u2r[0], rr[0], yr[1]);
+    load(i1 - 2 * CH, yr[0], ur[0], u2r[0], rr[0]);
+    back(i1 - CH, yr[1], ur[1], u2r[1], rr[1], yr[0]);
   }
   const double sc = s2 > 0.0 ? 1.0 / sqrt(s2) : 0.0;
-  for (int i0 = 0; i0 < n; i0 += kIvChunk) {
-    double xr[kIvChunk];
+  constexpr int CS = 64;
+  for (int i0 = 0; i0 < n; i0 += CS) {
+    double xs[CS];
 #pragma unroll
-    for (int c = 0; c < kIvChunk; ++c)
-      if (i0 + c < n) xr[c] = L_(x, i0 + c);
+    for (int c = 0; c < CS; ++c) xs[c] = L_(x, min(i0 + c, n - 1));
 #pragma unroll
-    for (int c = 0; c < kIvChunk; ++c)
-      if (i0 + c < n) L_(x, i0 + c) = xr[c] * sc;
+    for (int c = 0; c < CS; ++c)
+      if (i0 + c < n) L_(x, i0 + c) = xs[c] * sc;
   }
 #undef L_
 }
@@ -968,8 +992,9 @@ int dense_eigh(Ctx* c, double* a, int n, double* z, double* w, double* work, int
   const dim3 tgrid((n + 31) / 32, (n + 31) / 32);
   for (int pass = 0; pass < 2; ++pass) {
     if (pass > 0) hipLaunchKernelGGL(k_transpose_sq, tgrid, dim3(256), 0, st, z, n, X);
-    hipLaunchKernelGGL(k_inviter_par, dim3((n + 63) / 64), dim3(64), 0, st, d, e, n, w, bounds, lu,
-                       X, pass == 0 ? 1 : 0);
+    hipLaunchKernelGGL((n <= kBisectLds ? k_inviter_par<true> : k_inviter_par<false>),
+                       dim3((n + 63) / 64), dim3(64), 0, st, d, e, n, w, bounds, lu, X,
+                       pass == 0 ? 1 : 0);
     hipLaunchKernelGGL(k_transpose_sq, tgrid, dim3(256), 0, st, X, n, z);
     if (local) {
       hipLaunchKernelGGL(k_cluster_orth, dim3(n), dim3(256), 0, st, z, n, cl);
