@@ -2,8 +2,9 @@
 //
 //   * Cholesky S = L L^T and the explicit inverse L^-1 (the role of rsdecmp /
 //     rsinvcd, Sources/schmidt.f90:428-544) with the positive-definite check of
-//     schmidt2 (Sources/schmidt.f90:256-267), blocked by 64: the diagonal block
-//     is factored and inverted in LDS, the panel below and the trailing matrix
+//     schmidt2 (Sources/schmidt.f90:256-267): one workgroup up to order 192
+//     (dense_small.hip), else blocked by 64: the diagonal block is factored and
+//     inverted in the registers of one workgroup, the panel below and the trailing matrix
 //     are updated by many workgroups, and L^-1 is assembled block row by block
 //     row, X_ij = -X_ii sum_{k=j}^{i-1} L_ik X_kj.
 //   * The symmetric eigenproblem of the subspace Hamiltonian (the role of
@@ -238,8 +239,8 @@ __global__ void k_flag_to_ok(const int* fail, int* ok) { ok[0] = fail[0] ? 0 : 1
 // diagonal block: P (lower part filled, in LDS) -> X_bb = L_bb^-1 (the full block,
 // zeros above), factored in the registers of the workgroup: 64 steps of one
 // barrier each.  With the block in LDS and three barriers a step this was most
-// of the time of a block column; n = 540: 943 -> 427 us  fail[0] = 1 where a
-// pivot is not positive (dg = 0: no rounding bound, the pivots are those of a
+// of the time of a block column; n = 540, with the tile loads of coop.h
+// issued together: 943 -> 427 us.  fail[0] = 1 where a pivot is not positive (dg = 0: no rounding bound, the pivots are those of a
 // Schur complement).
 __device__ inline void chol_diag_block(int n, int k0, int kb, double* x, int* fail,
                                        double (*P)[NBK + 1]) {

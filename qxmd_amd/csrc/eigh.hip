@@ -2,7 +2,8 @@
 // (the role of RsEIGQR, Sources/funcs.f90:380-764: eigenvalues ascending with
 // their vectors), built for many workgroups:
 //
-//   1. Householder tridiagonalisation in one cooperative launch: the rows of
+//   1. Householder tridiagonalisation, up to order 192 in one workgroup
+//      (dense_small.hip), else in one cooperative launch: the rows of
 //      A live in the LDS of the workgroups (row i in workgroup i mod G); each
 //      step publishes a column, every workgroup forms the reflector from it,
 //      the row owners form p = A v and publish it, and every workgroup applies

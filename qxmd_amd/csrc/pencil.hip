@@ -9,6 +9,8 @@
 //   plane  : per z-plane, inverse y (pruned to |h| <= hmax), inverse x, x V(r),
 //            forward x, forward y, all in LDS                         -> T2
 //   zfwd   : forward FFT along z, split the two bands, x1/N, add |G|^2 psi.
+// Grids whose edges all have a two-step transform run pencil_fast.hip; the
+// Stockham kernels here take the others.
 // T1/T2 hold only the columns the sphere touches ([bp][z][col]), so the HBM
 // stream per band pair is a few times the sphere size instead of the grid.
 #include <algorithm>
