@@ -239,9 +239,9 @@ __global__ void k_flag_to_ok(const int* fail, int* ok) { ok[0] = fail[0] ? 0 : 1
 // diagonal block: P (lower part filled, in LDS) -> X_bb = L_bb^-1 (the full block,
 // zeros above), factored in the registers of the workgroup: 64 steps of one
 // barrier each.  With the block in LDS and three barriers a step this was most
-// of the time of a block column; n = 540, with the tile loads of coop.h
-// issued together: 943 -> 427 us.  fail[0] = 1 where a pivot is not positive (dg = 0: no rounding bound, the pivots are those of a
-// Schur complement).
+// of the time of a block column; n = 540, with the tile loads of coop.h issued
+// together: 943 -> 427 us.  fail[0] = 1 where a pivot is not positive (dg = 0:
+// no rounding bound, the pivots are those of a Schur complement).
 __device__ inline void chol_diag_block(int n, int k0, int kb, double* x, int* fail,
                                        double (*P)[NBK + 1]) {
   using S = Shape<256, NBK / 16>;

@@ -459,10 +459,15 @@ int kp_local_fast(Ctx* c, KFastArgs a, int nH, const double* src, double* dst, d
   const EdgeKernels<double> kz = edge_kernels<double>(c->n3);
   const auto plane = edge_kernels<double>(c->n1).kplane[s.yk];
   if (!kz.kzinv || !kz.kzfwd || !plane) return -3;
-  // as many wavefronts as the x pass has row groups for, 4 or 8 (small cells:
-  // 30 x 30 planes have three groups of ten rows)
+  // 8 wavefronts a block, 4 where the x pass has no more than four row groups.
+  // Where the launch has blocks enough and six fit a CU, two: the other blocks
+  // fill the time at the barriers, and no wavefront waits for a last row group
+  // (30 x 30 planes have three; 64 k-points x 20 bands there, whole H|psi>: 379 us
+  // with 4, 362 with 3, 343 with 2, 341 with 1).
   int nwave = plane_waves(s);
   if (nwave == 8 && (s.n2 + s.rw - 1) / s.rw <= 4) nwave = 4;
+  if (nwave == 4 && (long)c->n3 * nkb >= 4096 && 6 * s.lds(s.n2, s.n1, 2) <= kCuLds)
+    nwave = 2;
   if (nwave < 1) return -3;
   FastArgs f = fast_args(c, s, 0, 0);
   plane_strides(s, nwave, &f.sa, &f.sr);
