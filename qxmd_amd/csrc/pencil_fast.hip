@@ -462,8 +462,8 @@ int kp_local_fast(Ctx* c, KFastArgs a, int nH, const double* src, double* dst, d
   // 8 wavefronts a block, 4 where the x pass has no more than four row groups.
   // Where the launch has blocks enough and six fit a CU, two: the other blocks
   // fill the time at the barriers, and no wavefront waits for a last row group
-  // (30 x 30 planes have three; 64 k-points x 20 bands there, whole H|psi>: 379 us
-  // with 4, 362 with 3, 343 with 2, 341 with 1).
+  // (30 x 30 planes have three; 64 k-points x 20 bands there: 243 -> 193 us; whole
+  // H|psi> with 4, 3, 2, 1 wavefronts: 379, 362, 343, 341 us).
   int nwave = plane_waves(s);
   if (nwave == 8 && (s.n2 + s.rw - 1) / s.rw <= 4) nwave = 4;
   if (nwave == 4 && (long)c->n3 * nkb >= 4096 && 6 * s.lds(s.n2, s.n1, 2) <= kCuLds)
