@@ -9,9 +9,11 @@
 // both, d the pivot, with src = column k right of k, row k left of it and 1 at
 // it (where A(i, k) itself starts from 0).  Lower triangle only.
 //
-// A pivot counts as positive when it is above the rounding error of its own
-// sum, 8 eps S(k, k): of two equal bands the second one's pivot is a rounding
-// residue of either sign.
+// A pivot counts as positive above 1e-30, the guard of rsdecmp, at every order.
+// The quotients A(i, k) / d are corrected by their remainder, so that an A(i, k)
+// equal to d gives one: the rows of two equal bands held here then stay equal,
+// and the second one's pivot is zero or negative, never a positive rounding
+// residue (n = 160: 111 us with these two FMAs a row and without).
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -26,7 +28,7 @@ struct Shape {
 
 template <class S>
 struct CholLds {
-  double src[2][S::NM], piv[2], dg[S::NM], inv[S::NM];
+  double src[2][S::NM], piv[2], inv[S::NM];
 };
 
 template <class S, int P>
@@ -40,20 +42,21 @@ __device__ inline void chol_phase(double (&A)[S::NR][S::NC], CholLds<S>& L, int 
     const double* src = L.src[q];
     double* nsrc = L.src[q ^ 1];
     __syncthreads();
-    const double d = L.piv[q], dgk = L.dg[k];
+    const double d = L.piv[q];
     double l[NR], u[NC];
 #pragma unroll
     for (int r = R0; r < NR; ++r) l[r] = src[ti + RW * r];
 #pragma unroll
     for (int c = 0; c < NC; ++c) u[c] = src[tj + 16 * c];
-    const bool pos = d > fmax(1e-30, 8.0 * 2.220446049250313e-16 * dgk);
+    const bool pos = d > 1e-30;
     good = good && pos;
     const double id = pos ? 1.0 / d : 0.0;
     if (t == 0) L.inv[k] = id;
     const bool mine = tj == (k & 15);
 #pragma unroll
     for (int r = R0; r < NR; ++r) {
-      l[r] *= -id;
+      const double w = l[r] * id;
+      l[r] = -fma(fma(-w, d, l[r]), id, w);
       if (r <= RM) l[r] = ti + RW * r > k ? l[r] : 0.0;
       A[r][P] = mine && (r > RM || ti + RW * r > k) ? 0.0 : A[r][P];
     }

@@ -240,8 +240,7 @@ __global__ void k_flag_to_ok(const int* fail, int* ok) { ok[0] = fail[0] ? 0 : 1
 // zeros above), factored in the registers of the workgroup: 64 steps of one
 // barrier each.  With the block in LDS and three barriers a step this was most
 // of the time of a block column; n = 540, with the tile loads of coop.h issued
-// together: 943 -> 427 us.  fail[0] = 1 where a pivot is not positive (dg = 0:
-// no rounding bound, the pivots are those of a Schur complement).
+// together: 943 -> 427 us.  fail[0] = 1 where a pivot is not positive.
 __device__ inline void chol_diag_block(int n, int k0, int kb, double* x, int* fail,
                                        double (*P)[NBK + 1]) {
   using S = Shape<256, NBK / 16>;
@@ -254,10 +253,7 @@ __device__ inline void chol_diag_block(int n, int k0, int kb, double* x, int* fa
     for (int c = 0; c < S::NC; ++c) {
       const int i = ti + S::RW * r, j = tj + 16 * c;
       A[r][c] = (i < kb && j < kb) ? P[max(i, j)][min(i, j)] : 0.0;
-      if (j == 0) {
-        L.src[0][i] = i == 0 ? 1.0 : A[r][c];
-        L.dg[i] = 0.0;
-      }
+      if (j == 0) L.src[0][i] = i == 0 ? 1.0 : A[r][c];
     }
   if (t == 0) L.piv[0] = A[0][0];
   bool good = true;

@@ -63,7 +63,6 @@ __global__ void __launch_bounds__(S::T) k_chol_inv_wg(const double* __restrict__
     for (int c = 0; c < S::NC; ++c) {
       const int i = ti + S::RW * r, j = tj + 16 * c;
       A[r][c] = (i < n && j < n) ? s[(size_t)max(i, j) + (size_t)n * min(i, j)] : 0.0;
-      if (i == j) L.dg[i] = A[r][c];
       if (j == 0) L.src[0][i] = i == 0 ? 1.0 : A[r][c];
     }
   if (t == 0) L.piv[0] = A[0][0];
