@@ -266,10 +266,12 @@ static std::vector<std::pair<int, int>> plane_stride_ranks(const PlaneShape& s, 
 }
 
 // the model's stride pair (QX_PLANE_SA / QX_PLANE_SR override), kept per shape
+// (all that the ranking reads: an n x n plane of a cube, of which yk is Y_CUBE,
+// has one twiddle table in LDS, that of a slab two)
 static void plane_strides(const PlaneShape& s, int nwave, int* psa, int* psr) {
   static std::mutex mu;
-  static std::map<std::array<int, 5>, std::pair<int, int>> cache;
-  const std::array<int, 5> key{s.n1, s.n2, s.nH, (int)s.elem, nwave};
+  static std::map<std::array<int, 6>, std::pair<int, int>> cache;
+  const std::array<int, 6> key{s.n1, s.n2, s.yk, s.nH, (int)s.elem, nwave};
   {
     std::lock_guard<std::mutex> lk(mu);
     auto it = cache.find(key);

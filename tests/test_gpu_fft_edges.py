@@ -66,3 +66,30 @@ def test_local_and_density_on_edges(nd):
         assert np.abs(got[p] - ref).max() < tol * np.abs(ref).max()
         assert np.abs(rho[p] - rref).max() < tol * np.abs(rref).max()
         assert np.array_equal(rho0[p], rho[p])  # the density does not need a potential
+
+
+@pytest.mark.parametrize("e", [100, 112])
+def test_two_step_density_after_a_cube(e, monkeypatch):
+    """e x e planes of a cube and of a slab have rows of their own strides (a slab
+    keeps a second twiddle table in LDS): after the cube, the slab's FP64 density
+    still runs on the two-step kernels, whose rounding is not that of the Stockham
+    lines."""
+    occ = np.array([2.0])
+    rho = {}
+    for nd in ((e, e, e), (e, e, 16)):
+        print("edges", nd, flush=True)
+        gs = pw.GSphere(np.diag([2 * np.pi * (n / 4.0 - 0.3) / np.sqrt(20.0) for n in nd]))
+        gs.nd, gs.N = nd, int(np.prod(nd))
+        psi = np.random.default_rng(e).standard_normal((1, 2 * (gs.nplw + 1)))
+        psi[:, 1] = 0.0
+        ctx = pw.PlaneWave(gs, 1)
+        try:
+            ctx.put(0, psi)
+            rho["two-step"] = ctx.density(0, 1, occ, 1.0)
+            monkeypatch.setenv("QX_GENERIC_FFT", "1")
+            rho["Stockham"] = ctx.density(0, 1, occ, 1.0)
+            monkeypatch.delenv("QX_GENERIC_FFT")
+        finally:
+            ctx.close()
+        assert np.abs(rho["two-step"] - rho["Stockham"]).max() < 1e-12 * rho["Stockham"].max()
+        assert not np.array_equal(rho["two-step"], rho["Stockham"])
