@@ -415,7 +415,7 @@ int gs_gemm_nn(Ctx* c, int M, int N, int K, double alpha, const double* A, int l
                int ldb, double beta, double* C, int ldc, int prec, int batch = 1, long sA = 0,
                long sB = 0, long sC = 0);
 // the same contractions with a precision: PREC_FP32 -> FP32 MFMA (operands
-// rounded to FP32, FP32 accumulation per K chunk), otherwise FP64
+// rounded to FP32, FP32 accumulation per K chunk of about 1024), otherwise FP64
 int gemm_tn_p(Ctx* c, int M, int N, int K, double alpha, const double* A, int lda,
               const double* B, int ldb, double beta, double* C, int ldc, int corr, int prec);
 int gemm_nn_p(Ctx* c, int M, int N, int K, double alpha, const double* A, int lda,

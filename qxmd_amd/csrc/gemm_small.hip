@@ -391,7 +391,6 @@ __global__ void __launch_bounds__(64, 2)
 }
 
 constexpr int kTarget = 512;  // workgroups of a launch with K slices (2 per CU)
-constexpr size_t kWsDoubles = (size_t)kTarget * 64 * 64;
 
 // the K-slice partials: kept by the context, grown to what its products need
 double* workspace(Ctx* c, size_t n) {
@@ -421,10 +420,18 @@ int launch_tn(Ctx* c, GsArgs g, int batch, int target, int kmin, const double* A
   // (a multiple of 8 of them stays one: trailing slices may be empty)
   int ks = (int)std::min<long>(target / ((long)tiles * batch), g.K / (kmin * KH));
   ks = std::max(1, ks >= 8 ? ks & ~7 : ks);
-  const size_t ws = (size_t)tiles * batch * ks * TM * TN;
-  if (ws > kWsDoubles) ks = 1;
-  double* W = ks > 1 ? workspace(c, ws) : nullptr;
-  if (!W) ks = 1;
+  // FP32 chains: a wavefront sums in FP32, the wavefronts' and the slices' sums are
+  // added in FP64.  The error grows with the chain (2080 x 100 x 13134, random
+  // operands: 9.9e-7 of the result with 3284 k a chain, 5.1e-7 with 832; of one
+  // sign 4.1e-7 and 1.1e-7), so a chain takes 1024 k at most, more only where the
+  // output alone is many of 2048 blocks of 64 x 64 (27 MB of partials at most)
+  if constexpr (sizeof(T) == 4) {
+    const long blocks = (long)cdivu(g.M, 64) * cdivu(g.N, 64);
+    const long chains = std::min<long>(cdivu(g.K, 1024), std::max(1L, 2048 / blocks));
+    ks = std::max(ks, (int)cdivu(chains, KH));
+  }
+  double* W = ks > 1 ? workspace(c, (size_t)tiles * batch * ks * TM * TN) : nullptr;
+  if (!W) ks = 1;  // one slice, or out of memory
   g.kper = (int)cdivu(cdivu(g.K, ks), 16 * KH) * 16 * KH;
   g.ks = ks;
   const dim3 grid(g.ks, tiles, batch);

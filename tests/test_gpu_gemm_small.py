@@ -48,3 +48,32 @@ def test_kb_shapes(npj, nb):
         assert np.abs(sl[:, :, 0] - p).max() < 1e-13 * np.abs(p).max()
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("npj,nb", [(5500, 32), (3648, 192)])
+def test_fp32_chains(si64, npj, nb):
+    """FP32 products are added in FP32 over about 1024 k and from there in FP64.
+    The products are 1.5 + 2^-13 x bit: sums of up to 1365 of them stay below 2048,
+    where FP32 holds every multiple of 2^-13, so the projection is exact and the
+    back-projection gets it rounded to FP32 once; longer chains round on the way.
+    Outputs with tiles enough (of 32 x 32 and of 64 x 64) to leave K in one or
+    two slices by their number alone."""
+    print("FP32 chains", npj, nb, flush=True)
+    n = si64.nplwex
+    rng = np.random.default_rng(7)
+    psi = 1.5 + 2.0 ** -13 * rng.integers(0, 2, (nb, n))
+    psi[:, 1] = 0.0
+    ctx = pw.PlaneWave(pw.GSphere(si64.cell.hcell), nb)
+    try:
+        ctx.set_glocal(np.zeros(ctx.gs.N))
+        ctx.put(0, psi)
+        p = 2.0 * psi.sum(1) - psi[:, 0]
+        ref = psi * np.repeat(ctx.gs.recnrm[: n // 2], 2) + p.astype(np.float32)[:, None]
+        d = np.zeros((npj, 1))
+        d[npj - 1] = 1.0  # the one projector that counts
+        ctx.set_kb(np.ones((npj, 1, n)), np.ones(npj, np.int32), d)
+        ctx.hpsi(0, 1, nb, pw.MIXED)
+        # FP64 roundings of sums below 65536
+        assert np.abs(ctx.get(1, nb) - ref).max() < 1e-10
+    finally:
+        ctx.close()
