@@ -462,12 +462,18 @@ int tn(Ctx* c, const GsArgs& g, int batch, const double* A, const double* B, dou
   // 64 x 32 tiles where they are full (256 x 160 x 13134: 31 against 43); for
   // FP32, whose MFMAs ask for operands twice as fast, 64 x 64 on large outputs
   // (384 x 240 x 19588 FP32: 79 against 83, 256 x 160 x 13134 FP32: 34 against 28)
-  if (std::min(g.M, g.N) >= 128) {
-    if constexpr (sizeof(T) == 4)
-      if ((long)g.M * g.N >= 65536)
-        return launch_tn<T, 4, 4, 1, 1, 4, 1>(c, g, batch, kTarget, 64, A, B, C);
-    return launch_tn<T, 4, 2, 1, 1, 4, 1>(c, g, batch, kTarget, 64, A, B, C);
+  // and, from 2^30 products on, for all that does not fit one tile of 32: each
+  // column of tiles reads the long operand from memory again (both products of a
+  // KB term, 32 x 32 and 64 x 64: 864 x 64 x 43820 358 and 255, 2000 x 127 x 43820
+  // 1262 and 829, 700 x 127 x 13134 154 and 128; below the line 256 x 127 x 13134
+  // 58 and 63, 500 x 127 x 1648 33 and 36)
+  if constexpr (sizeof(T) == 4) {
+    const long lo = std::min(g.M, g.N), mn = (long)g.M * g.N;
+    if ((lo >= 128 && mn >= 65536) || (lo > 32 && mn * g.K >= 1L << 30))
+      return launch_tn<T, 4, 4, 1, 1, 4, 1>(c, g, batch, kTarget, 64, A, B, C);
   }
+  if (std::min(g.M, g.N) >= 128)
+    return launch_tn<T, 4, 2, 1, 1, 4, 1>(c, g, batch, kTarget, 64, A, B, C);
   return launch_tn<T, 2, 2, 1, 1, 4, 2>(c, g, batch, kTarget, 64, A, B, C);
 }
 

@@ -50,6 +50,32 @@ def test_kb_shapes(npj, nb):
         ctx.close()
 
 
+@pytest.mark.parametrize("npj,nb", [(2043, 40), (2046, 40), (1241, 66), (651, 127)])
+def test_kb_long(si64, npj, nb):
+    """The mixed KB term on both sides of 2^30 products, where 64 x 64 tiles take
+    over from 32 x 32 ones.  Two FP32 products of operands rounded to FP32:
+    sqrt(13134) 6e-8 = 6.9e-6 of the largest value."""
+    print("KB term", npj, "projectors", nb, "bands", flush=True)
+    n = si64.nplwex
+    rng = np.random.default_rng(npj)
+    psi = rng.standard_normal((nb, n))
+    psi[:, 1] = 0.0
+    b = rng.standard_normal((npj, n))
+    d = rng.standard_normal((npj, 1))
+    p = 2.0 * psi @ b.T - np.outer(psi[:, 0], b[:, 0])
+    ref = (p * d[:, 0]) @ b
+    ctx = pw.PlaneWave(pw.GSphere(si64.cell.hcell), nb)
+    try:
+        ctx.set_glocal(np.zeros(ctx.gs.N))
+        ctx.put(0, psi)
+        ctx.set_kb(b[:, None, :], np.ones(npj, np.int32), d)
+        ctx.hpsi(0, 1, nb, pw.MIXED)
+        got = ctx.get(1, nb) - psi * np.repeat(ctx.gs.recnrm[: n // 2], 2)
+        assert np.abs(got - ref).max() < 6.9e-6 * np.abs(ref).max()
+    finally:
+        ctx.close()
+
+
 @pytest.mark.parametrize("npj,nb", [(5500, 32), (3648, 192)])
 def test_fp32_chains(si64, npj, nb):
     """FP32 products are added in FP32 over about 1024 k and from there in FP64.
