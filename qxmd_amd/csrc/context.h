@@ -404,9 +404,9 @@ struct HostRead {
 };
 int read_host(Ctx* c, std::initializer_list<HostRead> segs);
 double* call_workspace(Ctx* c, size_t n);
-// the products with a dimension of the output below 256 (gemm_small.hip), in
-// either precision, over `batch` operands at the given strides; rscale: a
-// factor per row m of C (TN)
+// the products with a dimension of the output below 256, and FP64 ones with an
+// odd leading dimension (gemm_small.hip), in either precision, over `batch`
+// operands at the given strides; rscale: a factor per row m of C (TN)
 int gs_gemm_tn(Ctx* c, int M, int N, int K, double alpha, const double* A, int lda, const double* B,
                int ldb, double beta, double* C, int ldc, int corr, int prec,
                const double* rscale = nullptr, int batch = 1, long sA = 0, long sB = 0,

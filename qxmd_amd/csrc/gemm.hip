@@ -15,8 +15,8 @@
 // which skips Im c(G=0): Sources/nlkbpp.f90:1360-1363).
 //
 // Sizable outputs (M, N >= 256) run on the 128 x 128 kernels of
-// mfma_gemm.hip, smaller ones on gemm_small.hip, at most 4 columns on the
-// matrix-vector kernels here.
+// mfma_gemm.hip, smaller ones (and FP64 ones with an odd leading dimension) on
+// gemm_small.hip, at most 4 columns on the matrix-vector kernels here.
 #include <algorithm>
 #include <atomic>
 #include <cstdlib>

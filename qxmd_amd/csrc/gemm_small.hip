@@ -1,6 +1,9 @@
 // gemm_small.hip -- the contractions of gemm.hip whose output has fewer than
 // 256 rows or columns: small cells, CG blocks of a few bands, the k-points of
 // a mesh (batched).  FP64, or the mixed form's FP32 MFMA on FP64 operands.
+// FP64 products of any size come here too when a leading dimension is odd, which
+// the 16-byte rows of mfma_gemm.hip exclude (psi L^-T and the rotation of an odd
+// number of bands; Gram-Schmidt of 541 bands of 43820 1.39 ms, of 540 1.24).
 //
 // What bounds these is latency and occupancy, not the matrix cores: 32 x 20
 // outputs of 1648 plane waves are four MFMA tiles with one long sum each.  So
@@ -99,22 +102,21 @@ __device__ inline void load2(const double* p, double (&r)[2]) {
 // C(m, n) = alpha sum_k A[m][k] B[n][k] ... : blockIdx.x K slice (fastest, so
 // that a slice count divisible by 8 keeps a slice's workgroups on one XCD and
 // its operand columns in one L2), blockIdx.y tile, blockIdx.z batch.
-// BI x BJ blocks of 16 along m and n per wavefront, WM x WN wavefronts per
-// tile, KH groups of them sharing the slice 16 k at a time.
-template <typename T, bool VEC, int BI, int BJ, int WM, int WN, int KH, int DP>
-__global__ void __launch_bounds__(64 * WM * WN * KH, KH == 16 ? 1 : 2)
+// BI x BJ blocks of 16 along m and n; the KH wavefronts of a workgroup share the
+// slice 16 k at a time.
+constexpr int KH = 4;
+template <typename T, bool VEC, int BI, int BJ, int DP>
+__global__ void __launch_bounds__(64 * KH, 2)
     k_gs_tn(GsArgs g, const double* __restrict__ A0, const double* __restrict__ B0,
             double* __restrict__ C0, double* __restrict__ Wp) {
-  constexpr int TM = 16 * BI * WM, TN = 16 * BJ * WN;
+  constexpr int TM = 16 * BI, TN = 16 * BJ;
   typedef typename Mma<T>::acc_t acc_t;
-  __shared__ T red[KH][KH > 1 ? WM * WN * BI * BJ * 4 : 1][64];
+  __shared__ T red[KH][BI * BJ * 4][64];
   const double* A = A0 + (size_t)blockIdx.z * g.sA;
   const double* B = B0 + (size_t)blockIdx.z * g.sB;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int wt = wave % (WM * WN), kh = wave / (WM * WN);
+  const int lane = threadIdx.x & 63, kh = threadIdx.x >> 6;
   const int tile = (int)blockIdx.y;
-  const int m0 = (tile % g.tiles_m) * TM + (wt % WM) * 16 * BI;
-  const int n0 = (tile / g.tiles_m) * TN + (wt / WM) * 16 * BJ;
+  const int m0 = (tile % g.tiles_m) * TM, n0 = (tile / g.tiles_m) * TN;
   const int r = lane & 15, q = lane >> 4;
   const int kb = (int)blockIdx.x * g.kper, ke = min(g.K, kb + g.kper);
   const double *pa[BI], *pb[BJ];
@@ -178,41 +180,26 @@ __global__ void __launch_bounds__(64 * WM * WN * KH, KH == 16 ? 1 : 2)
   const size_t slot = ((size_t)blockIdx.z * gridDim.y + tile) * g.ks + blockIdx.x;
   double* P = Wp + slot * (TM * TN);
   double* C = C0 + (size_t)blockIdx.z * g.sC;
-  const int mt = (tile % g.tiles_m) * TM, nt = (tile / g.tiles_m) * TN;
-  auto store = [&](int ml, int nl, double s) {  // C or partial (mt + ml, nt + nl)
-    const int m = mt + ml, n = nt + nl;
+  // every wavefront leaves its sums in LDS and adds up its share of the tile
+  constexpr int ROWS = BI * BJ * 4;
+#pragma unroll
+  for (int i = 0; i < BI; ++i)
+#pragma unroll
+    for (int j = 0; j < BJ; ++j)
+#pragma unroll
+      for (int v = 0; v < 4; ++v) red[kh][(i * BJ + j) * 4 + v][lane] = acc[i][j][v];
+  __syncthreads();
+  for (int row = kh; row < ROWS; row += KH) {
+    double s = (double)red[0][row][lane];
+#pragma unroll
+    for (int h = 1; h < KH; ++h) s += (double)red[h][row][lane];
+    const int i = row / (4 * BJ), j = row / 4 % BJ, v = row % 4;
+    const int ml = 16 * i + r, nl = 16 * j + Mma<T>::row(lane, v), m = m0 + ml, n = n0 + nl;
     if (g.ks > 1) {
       P[nl * TM + ml] = s;
     } else if (m < g.M && n < g.N) {
       double* cp = C + (size_t)n * g.ldc + m;
       *cp = gs_value(g, s, A, B, cp, m, n);
-    }
-  };
-  if constexpr (KH == 1) {
-#pragma unroll
-    for (int i = 0; i < BI; ++i)
-#pragma unroll
-      for (int j = 0; j < BJ; ++j)
-#pragma unroll
-        for (int v = 0; v < 4; ++v)
-          store((wt % WM) * 16 * BI + 16 * i + r,
-                (wt / WM) * 16 * BJ + 16 * j + Mma<T>::row(lane, v), (double)acc[i][j][v]);
-  } else {
-    // every wavefront leaves its sums in LDS and adds up its share of the tile
-    constexpr int PW = BI * BJ * 4, ROWS = WM * WN * PW, W = WM * WN * KH;
-#pragma unroll
-    for (int i = 0; i < BI; ++i)
-#pragma unroll
-      for (int j = 0; j < BJ; ++j)
-#pragma unroll
-        for (int v = 0; v < 4; ++v) red[kh][wt * PW + (i * BJ + j) * 4 + v][lane] = acc[i][j][v];
-    __syncthreads();
-    for (int row = wave; row < ROWS; row += W) {
-      double s = (double)red[0][row][lane];
-#pragma unroll
-      for (int h = 1; h < KH; ++h) s += (double)red[h][row][lane];
-      const int w = row / PW, e = row % PW, i = e / (4 * BJ), j = e / 4 % BJ, v = e % 4;
-      store((w % WM) * 16 * BI + 16 * i + r, (w / WM) * 16 * BJ + 16 * j + Mma<T>::row(lane, v), s);
     }
   }
 }
@@ -391,6 +378,7 @@ __global__ void __launch_bounds__(64, 2)
 }
 
 constexpr int kTarget = 512;  // workgroups of a launch with K slices (2 per CU)
+constexpr int kMin = 64;      // least k of a wavefront
 
 // the K-slice partials: kept by the context, grown to what its products need
 double* workspace(Ctx* c, size_t n) {
@@ -410,15 +398,15 @@ double* workspace(Ctx* c, size_t n) {
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 
-template <typename T, int BI, int BJ, int WM, int WN, int KH, int DP>
-int launch_tn(Ctx* c, GsArgs g, int batch, int target, int kmin, const double* A, const double* B,
+template <typename T, int BI, int BJ, int DP>
+int launch_tn(Ctx* c, GsArgs g, int batch, int target, const double* A, const double* B,
               double* C) {
-  constexpr int TM = 16 * BI * WM, TN = 16 * BJ * WN;
+  constexpr int TM = 16 * BI, TN = 16 * BJ;
   g.tiles_m = (int)cdivu(g.M, TM);
   const int tiles = g.tiles_m * (int)cdivu(g.N, TN);
-  // K slices: enough workgroups for the chip, at least kmin k per wavefront
+  // K slices: enough workgroups for the chip, at least kMin k per wavefront
   // (a multiple of 8 of them stays one: trailing slices may be empty)
-  int ks = (int)std::min<long>(target / ((long)tiles * batch), g.K / (kmin * KH));
+  int ks = (int)std::min<long>(target / ((long)tiles * batch), g.K / (kMin * KH));
   ks = std::max(1, ks >= 8 ? ks & ~7 : ks);
   // FP32 chains: a wavefront sums in FP32, the wavefronts' and the slices' sums are
   // added in FP64.  The error grows with the chain (2080 x 100 x 13134, random
@@ -435,15 +423,14 @@ int launch_tn(Ctx* c, GsArgs g, int batch, int target, int kmin, const double* A
   g.kper = (int)cdivu(cdivu(g.K, ks), 16 * KH) * 16 * KH;
   g.ks = ks;
   const dim3 grid(g.ks, tiles, batch);
-  constexpr int threads = 64 * WM * WN * KH;
   const bool vec = !(g.lda & 1) && !(g.ldb & 1) && !(g.sA & 1) && !(g.sB & 1) && aligned16(A) &&
                    aligned16(B);
   if (vec)
-    hipLaunchKernelGGL((k_gs_tn<T, true, BI, BJ, WM, WN, KH, DP>), grid, dim3(threads), 0,
-                       c->stream, g, A, B, C, W);
+    hipLaunchKernelGGL((k_gs_tn<T, true, BI, BJ, DP>), grid, dim3(64 * KH), 0, c->stream, g, A, B,
+                       C, W);
   else
-    hipLaunchKernelGGL((k_gs_tn<T, false, BI, BJ, WM, WN, KH, DP>), grid, dim3(threads), 0,
-                       c->stream, g, A, B, C, W);
+    hipLaunchKernelGGL((k_gs_tn<T, false, BI, BJ, DP>), grid, dim3(64 * KH), 0, c->stream, g, A, B,
+                       C, W);
   if (g.ks > 1)
     hipLaunchKernelGGL(k_gs_fix, dim3(cdivu((long)g.M * g.N, 256), batch), dim3(256), 0, c->stream,
                        g, TM, TN, tiles, A, B, C, W);
@@ -458,7 +445,7 @@ int tn(Ctx* c, const GsArgs& g, int batch, const double* A, const double* B, dou
   // (32 x 20 x 1648: 8.4 against 11.5 on 32 x 32 tiles; 128 x 81 x 5222, 48
   // tiles: 11.9 against 11.4; 64 products of 64 x 20 x 1672: 27 against 22)
   const long t16 = (long)cdivu(g.M, 16) * cdivu(g.N, 16) * batch;
-  if (t16 <= 32) return launch_tn<T, 1, 1, 1, 1, 4, 4>(c, g, batch, 1024, 64, A, B, C);
+  if (t16 <= 32) return launch_tn<T, 1, 1, 4>(c, g, batch, 1024, A, B, C);
   // 64 x 32 tiles where they are full (256 x 160 x 13134: 31 against 43); for
   // FP32, whose MFMAs ask for operands twice as fast, 64 x 64 on large outputs
   // (384 x 240 x 19588 FP32: 79 against 83, 256 x 160 x 13134 FP32: 34 against 28)
@@ -470,11 +457,11 @@ int tn(Ctx* c, const GsArgs& g, int batch, const double* A, const double* B, dou
   if constexpr (sizeof(T) == 4) {
     const long lo = std::min(g.M, g.N), mn = (long)g.M * g.N;
     if ((lo >= 128 && mn >= 65536) || (lo > 32 && mn * g.K >= 1L << 30))
-      return launch_tn<T, 4, 4, 1, 1, 4, 1>(c, g, batch, kTarget, 64, A, B, C);
+      return launch_tn<T, 4, 4, 1>(c, g, batch, kTarget, A, B, C);
   }
   if (std::min(g.M, g.N) >= 128)
-    return launch_tn<T, 4, 2, 1, 1, 4, 1>(c, g, batch, kTarget, 64, A, B, C);
-  return launch_tn<T, 2, 2, 1, 1, 4, 2>(c, g, batch, kTarget, 64, A, B, C);
+    return launch_tn<T, 4, 2, 1>(c, g, batch, kTarget, A, B, C);
+  return launch_tn<T, 2, 2, 2>(c, g, batch, kTarget, A, B, C);
 }
 
 template <typename T, int G, int BJ, int DP>
