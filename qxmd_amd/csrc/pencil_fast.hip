@@ -461,14 +461,19 @@ int kp_local_fast(Ctx* c, KFastArgs a, int nH, const double* src, double* dst, d
   const EdgeKernels<double> kz = edge_kernels<double>(c->n3);
   const auto plane = edge_kernels<double>(c->n1).kplane[s.yk];
   if (!kz.kzinv || !kz.kzfwd || !plane) return -3;
-  // 8 wavefronts a block, 4 where the x pass has no more than four row groups.
-  // Where the launch has blocks enough and six fit a CU, two: the other blocks
-  // fill the time at the barriers, and no wavefront waits for a last row group
-  // (30 x 30 planes have three; 64 k-points x 20 bands there: 243 -> 193 us; whole
-  // H|psi> with 4, 3, 2, 1 wavefronts: 379, 362, 343, 341 us).
+  // 8 wavefronts a block, 4 where the x pass has no more than four row groups (36 x
+  // 36, 1280 (k, band) blocks, whole local part: 600 us with 8, 421 with 4).  Where
+  // it has two to four, the launch blocks enough and six fit a CU, two: the other
+  // blocks fill the time at the barriers, and fewer wavefronts wait for a last row
+  // group.  With 4 and 2 wavefronts, 1280 (k, band) blocks, us: 20^3 121, 98; 24^3
+  // 226, 146; 28^3 272, 238; 30^3 296, 240; 32^3 331, 277; 36^3 423, 409; at the
+  // line, 4100 planes: 40, 37; 55, 44; 59, 55; 59, 54; 64, 59; 65, 63; at half of
+  // it: 31, 28; 38, 32; 41, 40; 41, 37; 43, 40; 46, 47.  One row group (16^3): 77, 81
   int nwave = plane_waves(s);
-  if (nwave == 8 && (s.n2 + s.rw - 1) / s.rw <= 4) nwave = 4;
-  if (nwave == 4 && (long)c->n3 * nkb >= 4096 && 6 * s.lds(s.n2, s.n1, 2) <= kCuLds)
+  const int groups = (s.n2 + s.rw - 1) / s.rw;
+  if (nwave == 8 && groups <= 4) nwave = 4;
+  if (nwave == 4 && groups > 1 && groups <= 4 && (long)c->n3 * nkb >= 4096 &&
+      6 * s.lds(s.n2, s.n1, 2) <= kCuLds)
     nwave = 2;
   if (nwave < 1) return -3;
   FastArgs f = fast_args(c, s, 0, 0);
