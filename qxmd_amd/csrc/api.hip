@@ -893,7 +893,7 @@ int qx_kbnlpp_frc2_slot(qx_ctx* h, int slot, int nb, const double* occ, const do
                         const double* gy, const double* gz, double* fnlc) {
   Ctx* c = &h->c;
   if (slot < 0 || slot >= Ctx::kSlots || (slot >= 2 && slot <= 4))
-    return fail(-1, "qx_kbnlpp_frc2_slot: slot 0, 1 or 5 (2-4 hold the G-weighted bands)");
+    return fail(-1, "qx_kbnlpp_frc2_slot: slot 0, 1 or 5 (2-4 are work slots)");
   if (nb < 1 || nb > c->nbmax) return fail(-1, "qx_kbnlpp_frc2_slot: 1 <= nb <= nbmax");
   const int rc = kb_forces(c, c->d_slot[slot], nb, occ, gx, gy, gz, fnlc);
   if (rc) return fail(rc, "qx_kbnlpp_frc2_slot failed");

@@ -126,7 +126,7 @@ int kb_forces(Ctx* c, const double* psi, int nb, const double* occ_host, const d
   if (c->npj == 0 || c->natom == 0) return 0;
   const int n = c->nplwex, np = c->nplw + 1, npj = c->npj;
   if (nb < 1 || nb > c->nbmax) return -1;
-  if (psi == c->d_slot[2] || psi == c->d_slot[3] || psi == c->d_slot[4]) return -1;
+  if (psi == c->d_slot[2]) return -1;  // Y's place
   // projections slmir = 2 B^T psi - G0 terms
   int rc = gemm_tn(c, npj, nb, n, 2.0, c->d_B, n, psi, n, 0.0, c->d_P, npj, 2);
   if (rc) return rc;

@@ -25,8 +25,8 @@
 // sphere) and x, x V(r), forward x and y, and forward z with the kinetic term.
 // T holds only the columns of each sphere ([kb][z][column]), in place.  The
 // two-step transforms of pencil_fast.h take the grids they cover (64 k-points
-// x 20 bands on 30^3, with the nonlocal part: 3.41 -> 0.32 ms); the others run here, on Stockham lines in
-// LDS over dense planes:
+// x 20 bands on 30^3, with the nonlocal part: 3.41 -> 0.33 ms); the others run
+// here, on Stockham lines in LDS over dense planes:
 //   k_kzinv  : the column points -> z lines in LDS, inverse FFT along z  -> T
 //   k_kplane : per z plane, the columns into a dense plane in LDS, inverse y
 //              and x, x V(r), forward x and y, back to the columns        -> T

@@ -780,7 +780,6 @@ struct MgState {
   size_t ws_bytes = 0;
   // tuned workgroup count per (kind, M, N, K, lda, ldb)
   std::map<std::tuple<int, int, int, int, int, int>, int> grid;
-  // FP64 output tile per (kind, M, N, K, lda, ldb): index into the variants
   float* f32[4] = {};  // FP32 work buffers of the fused mixed band-apply
   size_t f32_len[4] = {};
   float* B32 = nullptr;  // FP32 copy of the KB table
@@ -923,7 +922,7 @@ bool tuning_off() {
 
 // schedule of a product (a code of make_sk): the candidates of
 // sched_candidates, timed on first use of a shape with `trial(code)` (which
-// writes a scratch output), then cached; untimed, stream-K on two
+// writes a scratch output), then cached; untimed, stream-K on per_cu_max
 // workgroups per CU; 0 on failure
 template <typename F>
 int choose_grid(Ctx* c, int kind, int M, int N, int K, int kt, int tm, int tn, int lda, int ldb,

@@ -1,7 +1,7 @@
 """Nonlocal forces where the projectors do not fit one set of weighted bands:
 contexts of few bands (rows of the force workspace, in two chunks), of fewer
-bands than projectors (a slot, in chunks) and of more, for one to twenty bands,
-against the oracle."""
+bands than projectors (a slot, in chunks) and of more, for one to twenty bands and
+for an odd number above 256, against the oracle."""
 import numpy as np
 import pytest
 
@@ -12,7 +12,8 @@ from qxmd_amd.system import initial_wavefunctions, model_kb_projectors
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("nbmax,nb", [(1, 1), (5, 5), (20, 20), (67, 20), (150, 20), (300, 20)])
+@pytest.mark.parametrize("nbmax,nb", [(1, 1), (5, 5), (20, 20), (67, 20), (150, 20), (300, 20),
+                                      (257, 257)])
 def test_kb_forces_rows(si64, nbmax, nb):
     print("forces", nbmax, nb, flush=True)
     gs, ctx, H, v = parity._setup(si64, nbmax)

@@ -1,7 +1,8 @@
 """The FP64 products that leave half of the work out, by Gram-Schmidt against the
 oracle: the overlap on and below the diagonal tiles, psi L^-T up to each tile's
 last column, at band counts on, below and above the edges of the 96 and 128
-tiles, with each work schedule, and the orthonormality of the result."""
+tiles, with each work schedule, and the orthonormality of the result.  Odd
+counts have the same overlap and take gemm_small.hip for psi L^-T."""
 import numpy as np
 import pytest
 
@@ -12,7 +13,7 @@ from qxmd_amd.system import initial_wavefunctions
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("nb", [256, 258, 286, 288, 290, 384, 386])
+@pytest.mark.parametrize("nb", [256, 257, 258, 286, 288, 289, 290, 384, 385, 386])
 def test_schmidt_tile_edges(si64, nb):
     print("schmidt", nb, flush=True)
     raw = initial_wavefunctions(si64, nb)
