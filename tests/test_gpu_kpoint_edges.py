@@ -46,3 +46,35 @@ def test_khpsi_local_on_edges(nd):
                 assert np.abs(ctx.kget(1, ik) - ref).max() < 1e-12 * np.abs(ref).max(), ik
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("e", [16, 20, 30, 36, 40])
+@pytest.mark.parametrize("over", [0, 1])
+def test_khpsi_local_many_blocks(e, over):
+    """(k, band) blocks just below and at 4096 planes, where the plane pass takes two
+    wavefronts a block on two to four row groups (20, 30, 36; 16 has one, 40 five)."""
+    nk = (4096 + e - 1) // e - 1 + over
+    print("edge", e, "blocks", nk, flush=True)
+    hcell = np.eye(3) * 2 * np.pi * (e / 4.0 - 0.3) / np.sqrt(20.0)
+    gs = pw.GSphere(hcell)
+    gs.nd, gs.N = (e, e, e), e ** 3
+    rng = np.random.default_rng(e)
+    v = rng.standard_normal(gs.N)
+    kf = rng.uniform(-0.5, 0.5, (nk, 3))
+    ctx = pw.PlaneWave(gs, 1)
+    try:
+        ctx.set_glocal(v)
+        ctx.kpoints_set(kf, 2 * np.pi * np.linalg.inv(hcell).T, 20.0, 1)
+        data = []
+        for ik in range(nk):
+            hkl, kin = ctx.kpoints_sphere(ik)
+            c = rng.standard_normal((1, len(kin))) + 1j * rng.standard_normal((1, len(kin)))
+            ctx.kput(0, ik, c)
+            data.append((c, hkl, kin))
+        ctx.khpsi(0, 1)
+        for ik in list(range(0, nk, 7)) + [nk - 1]:
+            c, hkl, kin = data[ik]
+            ref = OK.hk_apply(c, hkl, kin, v.reshape(e, e, e))
+            assert np.abs(ctx.kget(1, ik) - ref).max() < 1e-12 * np.abs(ref).max(), ik
+    finally:
+        ctx.close()
